@@ -42,6 +42,9 @@ HIP_SOURCES = {
     "noalloc.hip": [],
     "segments.hip": [],
 }
+# sources compiled in several parts (one object each, -DPAGANI_PART=k), side
+# by side: their kernel instantiations take minutes in one
+PARTS = {"genz_eval.hip": 6, "segments.hip": 3}
 CXX_SOURCES = {"rule.cpp": ["-O2", "-ffp-contract=off"],
                "mcubes_grid.cpp": ["-O2", "-ffp-contract=off"]}
 
@@ -102,10 +105,19 @@ def generate_tuning_table():
     return path
 
 
-def _compile_hip(src, extra):
-    obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
+def _compile_hip(src, extra, part=None):
+    name = os.path.splitext(src)[0] + ("" if part is None else f".{part}")
+    obj = os.path.join(BUILD, name + ".o")
+    if part is not None:
+        extra = [*extra, f"-DPAGANI_PART={part}"]
     _run([HIPCC, *HIP_FLAGS, "-I" + BUILD, *extra, "-c", os.path.join(CSRC, src), "-o", obj])
     return obj
+
+
+def _hip_jobs():
+    """(source, flags, part) of every object, the sources in parts first: they take longest."""
+    parts = [(s, HIP_SOURCES[s], k) for s, n in PARTS.items() for k in range(n)]
+    return parts + [(s, f, None) for s, f in HIP_SOURCES.items() if s not in PARTS]
 
 
 def _compile_cxx(src, extra):
@@ -119,7 +131,7 @@ def build_library(jobs=8):
     os.makedirs(BUILD, exist_ok=True)
     generate_tuning_table()
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
-        futs = [ex.submit(_compile_hip, s, f) for s, f in HIP_SOURCES.items()]
+        futs = [ex.submit(_compile_hip, *job) for job in _hip_jobs()]
         futs += [ex.submit(_compile_cxx, s, f) for s, f in CXX_SOURCES.items()]
         objs = [f.result() for f in futs]
     tmp = LIB + ".tmp"

@@ -156,10 +156,15 @@ int run_item_resume(pagani_batch* b, int w, const pagani_batch_item& it,
     if (rc != PAGANI_ENOMEM) set_error(b, pagani_ws_last_error(ws));
     return rc;
   }
+  // the regular loop holds a uniform start's widths as levels
+  const std::size_t k = it.init_k ? it.init_k : I::default_split(d);
+  pagani::phases::Levels lv{};
+  lv.on = 1;
+  for (int j = 0; j < d; ++j) lv.h0[j] = 1. / static_cast<double>(k);
   if (hipMemcpyAsync(ws->L[0].p, v.L[o.cur], d * n * sizeof(double), hipMemcpyDeviceToDevice,
                      ws->stream) != hipSuccess ||
-      hipMemcpyAsync(ws->H[0].p, v.H[o.cur], d * n * sizeof(double), hipMemcpyDeviceToDevice,
-                     ws->stream) != hipSuccess ||
+      pagani::phases::to_levels(ws->stream, d, n, v.H[o.cur], lv,
+                                reinterpret_cast<std::uint16_t*>(ws->H[0].p)) != hipSuccess ||
       (np && hipMemcpyAsync(ws->pest.p, v.pest, np * sizeof(double), hipMemcpyDeviceToDevice,
                             ws->stream) != hipSuccess)) {
     (void)hipGetLastError();
@@ -172,7 +177,7 @@ int run_item_resume(pagani_batch* b, int w, const pagani_batch_item& it,
   st.n = n;
   st.has_parents = o.has_parents;
   st.split = 0;
-  st.lv = pagani::phases::Levels{};
+  st.lv = lv;
   st.user_regions = 0;
   st.relerr = it.relerr_classification ? 1 : 0;
   st.epsrel = it.epsrel;
@@ -268,7 +273,7 @@ int run_segments(pagani_batch* b, const pagani_batch_item* items, std::size_t co
         // on the whole device (measured: 165 ms for the 8D items of the
         // 512-integral batch, 4 ms each on the regular loop)
         if (fam == PAGANI_GENZ_CORNER_PEAK && d >= 8) continue;
-        const std::size_t k = it.init_k ? it.init_k : (d < 5 ? 4 : (d <= 10 ? 2 : 1));
+        const std::size_t k = it.init_k ? it.init_k : I::default_split(d);
         std::size_t n = 1;
         bool fits = true;
         for (int j = 0; j < d && fits; ++j) {
@@ -310,7 +315,7 @@ int run_segments(pagani_batch* b, const pagani_batch_item* items, std::size_t co
         s.f = it.f;
         s.epsrel = it.epsrel;
         s.epsabs = it.epsabs;
-        s.init_k = it.init_k ? it.init_k : (d < 5 ? 4 : (d <= 10 ? 2 : 1));
+        s.init_k = it.init_k ? it.init_k : I::default_split(d);
         s.relerr = it.relerr_classification ? 1 : 0;
         sel.push_back(s);
         idx.push_back(i);

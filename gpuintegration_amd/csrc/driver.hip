@@ -299,8 +299,9 @@ std::uint64_t round_cap(const pagani_ws* ws, std::uint64_t n, std::uint64_t cap,
   if (ws->slices_override <= 0)
     if (const std::uint8_t* t = tuned_table(ws)) {
       int b = slice_bucket(n);
-      if (t[b] > 0) {
-        while (b + 1 < kSliceBuckets && t[b + 1] == t[b] &&
+      const int e = tuned_entry(t, b);
+      if (e > 0) {
+        while (b + 1 < kSliceBuckets && tuned_entry(t, b + 1) == e &&
                (std::uint64_t(1) << (b + 1)) <= cap)
           ++b;
         const std::uint64_t end = b + 1 < 64 ? (std::uint64_t(2) << b) - 1 : cap;
@@ -613,7 +614,7 @@ int integrate_impl(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double epsrel,
     // grown by the first finds every buffer at its size in the next
     ws->cur = 0;
     ws->split = false;
-    std::size_t k = init_k ? init_k : (d < 5 ? 4 : (d <= 10 ? 2 : 1));
+    std::size_t k = init_k ? init_k : default_split(d);
     // every width of the run is 1/k halved some number of times: H holds
     // that number, one uint16_t per axis and region (pagani_eval_args)
     ws->lv = ph::Levels{};

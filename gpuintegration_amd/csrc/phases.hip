@@ -61,6 +61,19 @@ __global__ void __launch_bounds__(256) k_uniform_split(int d, std::size_t k, std
   }
 }
 
+// The levels of a flat list's widths, each h0[j] halved some number of times.
+__global__ void __launch_bounds__(256) k_to_levels(int d, std::size_t n,
+                                                   const double* __restrict__ H, const Levels lv,
+                                                   std::uint16_t* __restrict__ out)
+{
+  const std::size_t t = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  for (int j = 0; j < d; ++j) {
+    const std::size_t o = static_cast<std::size_t>(j) * n + t;
+    out[o] = static_cast<std::uint16_t>(ilogb(lv.h0[j]) - ilogb(H[o]));
+  }
+}
+
 // Row `row` of a list's bounds along axis j at stride `stride`: lower bound
 // and width (from the level when lv.on), and the width's level.
 __device__ __forceinline__ void read_row(const double* __restrict__ L,
@@ -1164,6 +1177,14 @@ hipError_t uniform_split(hipStream_t s, int d, std::size_t k, std::size_t n, dou
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_uniform_split, grid_for(n, 256), dim3(256), 0, s, d, k, n,
                      1. / static_cast<double>(k), L, H, levels ? 1 : 0);
+  return hipGetLastError();
+}
+
+hipError_t to_levels(hipStream_t s, int d, std::size_t n, const double* H, const Levels& lv,
+                     std::uint16_t* out)
+{
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_to_levels, grid_for(n, 256), dim3(256), 0, s, d, n, H, lv, out);
   return hipGetLastError();
 }
 

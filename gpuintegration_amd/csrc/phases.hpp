@@ -109,6 +109,11 @@ struct Levels {
 hipError_t uniform_split(hipStream_t s, int d, std::size_t k, std::size_t n, double* L,
                          double* H, bool levels = false);
 
+// The widths H of a flat n-region list as levels: H[j*n + i] is lv.h0[j]
+// halved out[j*n + i] times.
+hipError_t to_levels(hipStream_t s, int d, std::size_t n, const double* H, const Levels& lv,
+                     std::uint16_t* out);
+
 // Device-resident loop variants (lists of at most kDevLoopMax regions):
 // fixed launch shapes for n_cap regions, the actual count and selections
 // read from the descriptors; a descriptor with run == 0 makes them no-ops.

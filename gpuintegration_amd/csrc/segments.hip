@@ -142,9 +142,11 @@ __device__ void run_item(const F& f0, const SegItem& it, const SegPtrs& p, std::
       const std::size_t t0 = b * 64 + lane;
       const bool live = t0 < n;
       const std::size_t t = live ? t0 : n - 1;
-      detail::eval_regions_wave<D, F, double>(f, p.L[cur], p.H[cur], nullptr, n, t, live, C.lows,
-                                              C.range, C.jac, C, 1, 0, lane, nullptr, p.est,
-                                              p.err0, p.dim);
+      constexpr bool kPairs = detail::has_pair_sums<F>::value;
+      detail::LoadedRow<kPairs ? D : 1> row(p.L[cur], p.H[cur], nullptr, n, t, C);
+      detail::eval_regions_wave<D, F, double, kPairs>(
+          f, p.L[cur], p.H[cur], nullptr, n, t, live, C.lows, C.range, C.jac, C, 1, 0, lane,
+          nullptr, &row, nullptr, p.est, p.err0, p.dim);
     }
     __syncthreads();
     // RefineError with the relerr flags, and the iteration's sums
@@ -353,10 +355,15 @@ __global__ void __launch_bounds__(kSegThreads)
   }
 }
 
-template <int D = PAGANI_MIN_DIM, class Fn>
+// The dimensions whose kernels this part of the source holds (PAGANI_PART,
+// see build.py).
+constexpr int kPartFirst[] = {PAGANI_MIN_DIM, 6, 8, PAGANI_GENZ_MAX_DIM + 1};
+constexpr int kFirstDim = kPartFirst[PAGANI_PART], kLastDim = kPartFirst[PAGANI_PART + 1] - 1;
+
+template <int D = kFirstDim, class Fn>
 hipError_t with_genz_dim(int d, Fn&& fn)
 {
-  if constexpr (D > PAGANI_GENZ_MAX_DIM) {
+  if constexpr (D > kLastDim) {
     return hipErrorInvalidValue;
   } else {
     if (d == D) return fn(std::integral_constant<int, D>{});
@@ -396,6 +403,47 @@ unsigned resident(unsigned grid)
 
 }  // namespace
 
+template <int Part>
+hipError_t launch_segments_part(hipStream_t s, int d, int family, const SegItem* items,
+                                std::uint32_t count, std::uint32_t* next, char* pool,
+                                std::size_t bytes, std::size_t S, unsigned grid,
+                                const pagani_eval_consts& C, std::size_t mem_total, int mem_model,
+                                SegOut* out);
+template <int Part>
+unsigned segment_grid_part(int d, int family, unsigned want);
+
+template <>
+hipError_t launch_segments_part<PAGANI_PART>(hipStream_t s, int d, int family,
+                                             const SegItem* items, std::uint32_t count,
+                                             std::uint32_t* next, char* pool, std::size_t bytes,
+                                             std::size_t S, unsigned grid,
+                                             const pagani_eval_consts& C, std::size_t mem_total,
+                                             int mem_model, SegOut* out)
+{
+  return with_genz_dim(d, [&](auto D) {
+    return with_genz_family(family, [&](auto F) {
+      constexpr int Dv = decltype(D)::value, Fv = decltype(F)::value;
+      hipLaunchKernelGGL((k_segments<Dv, Fv>), dim3(grid), dim3(kSegThreads), 0, s, items,
+                         count, next, pool, bytes, S, C, mem_total, mem_model, out);
+      return hipGetLastError();
+    });
+  });
+}
+
+template <>
+unsigned segment_grid_part<PAGANI_PART>(int d, int family, unsigned want)
+{
+  unsigned g = want;
+  (void)with_genz_dim(d, [&](auto D) {
+    return with_genz_family(family, [&](auto F) {
+      g = resident<decltype(D)::value, decltype(F)::value>(want);
+      return hipSuccess;
+    });
+  });
+  return g;
+}
+
+#if PAGANI_PART == 0
 std::size_t segment_bytes(int d, std::size_t regions) { return seg_bytes(d, regions); }
 
 SegView segment_view(char* base, int d, std::size_t regions)
@@ -416,27 +464,20 @@ hipError_t launch_segments(hipStream_t s, int d, int family, const SegItem* item
                            const pagani_eval_consts& C, std::size_t mem_total, int mem_model,
                            SegOut* out)
 {
-  return with_genz_dim(d, [&](auto D) {
-    return with_genz_family(family, [&](auto F) {
-      constexpr int Dv = decltype(D)::value, Fv = decltype(F)::value;
-      hipLaunchKernelGGL((k_segments<Dv, Fv>), dim3(grid), dim3(kSegThreads), 0, s, items,
-                         count, next, pool, bytes, S, C, mem_total, mem_model, out);
-      return hipGetLastError();
-    });
-  });
+  auto launch = d < kPartFirst[1]   ? &launch_segments_part<0>
+                : d < kPartFirst[2] ? &launch_segments_part<1>
+                                    : &launch_segments_part<2>;
+  return launch(s, d, family, items, count, next, pool, bytes, S, grid, C, mem_total, mem_model,
+                out);
 }
 
 unsigned segment_grid(int d, int family, unsigned want)
 {
-  unsigned g = want;
-  (void)with_genz_dim(d, [&](auto D) {
-    return with_genz_family(family, [&](auto F) {
-      g = resident<decltype(D)::value, decltype(F)::value>(want);
-      return hipSuccess;
-    });
-  });
-  return g;
+  return d < kPartFirst[1]   ? segment_grid_part<0>(d, family, want)
+         : d < kPartFirst[2] ? segment_grid_part<1>(d, family, want)
+                             : segment_grid_part<2>(d, family, want);
 }
+#endif
 
 }  // namespace internal
 }  // namespace pagani

@@ -52,11 +52,12 @@ def family_params(family, d, seed):
 
 
 def regions(d, n, seed, device):
-    """n random sub-boxes of the unit cube (SoA), widths 10^U(-3, -0.3)."""
+    """n random sub-boxes of the unit cube (SoA) with the widths a run's lists
+    hold: 1/2 to 1/1024, powers of two."""
     import torch
     gen = torch.Generator().manual_seed(seed)
-    H = 10.0 ** (-3.0 + 2.7 * torch.rand((d, n), generator=gen, dtype=torch.float64))
-    L = torch.rand((d, n), generator=gen, dtype=torch.float64) * (1.0 - H)
+    H = 0.5 ** torch.randint(1, 11, (d, n), generator=gen).to(torch.float64)
+    L = torch.floor(torch.rand((d, n), generator=gen, dtype=torch.float64) / H) * H
     return L.reshape(-1).contiguous().to(device), H.reshape(-1).contiguous().to(device)
 
 
@@ -90,7 +91,9 @@ def tune(dims, families, precisions, buckets, launches, log=print):
                     for prec in precisions:
                         t = {s: time_shape(ws, fam, a, u, n, L, H, est, err, dim, prec, s,
                                            launches) for s in SLICES}
-                        best = min(SLICES, key=lambda s: (t[s], s))
+                        # more waves per batch only where they are clearly
+                        # faster: launches differ by a few per cent
+                        best = min(s for s in SLICES if t[s] <= 1.04 * min(t.values()))
                         row = next((r for r in tables if r["family"] == fam and r["ndim"] == d
                                     and r["precision"] == prec), None)
                         if row is None:

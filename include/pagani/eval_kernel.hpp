@@ -164,6 +164,36 @@ template <class F>
 struct has_axis_aux<F, std::void_t<decltype(std::declval<const F&>().axis_aux(0, 0.0))>>
     : std::true_type {};
 
+// Factored integrands whose value depends on a +-pair of points of one axis
+// only through the pair's sum may give the five sums themselves: `void
+// pair_sums(int j, double c, double h, const double* w, const double* table,
+// double (&s)[5])`, s[i] = (f at c - l_i h on axis j + f at c + l_i h) / (f
+// at c) for l_0..l_4 = lambda1..lambda5 (masked points count as zero).  Every
+// rule sum and every fourth difference is a function of these sums alone, so
+// nothing else of the pair is formed.  w holds the kWidthValues values
+// `width_values(double a, double (&w)[kWidthValues])` gives for a =
+// `width_arg(int j, double h)`, the functions of the axis' width alone; table holds kTableSize doubles in LDS
+// (`fill_table(double*, int tid, int threads)`), or is NULL.  The nested type Centre
+// collects the axes' centres (add(f, j, c, h)), says whether the sums and
+// their products stay in range (safe(f)) and gives the centre's value up to
+// value() (value(f)).
+template <class F, class = void>
+struct has_pair_sums : std::false_type {};
+template <class F>
+struct has_pair_sums<F, std::void_t<decltype(std::declval<const F&>().pair_sums(
+                            0, 0.0, 0.0, nullptr, nullptr, std::declval<double (&)[5]>()))>>
+    : std::true_type {};
+
+// Additive integrands (term, outer) may give outer summed over the points of
+// a group: `double sum2(s0, s1)`, `double sum4(s0, s1, s2, s3)`, with `bool
+// sum_safe(const double (&c)[D], const double (&h)[D])` true where every
+// point of a region with centre c and widths h may be summed so.
+template <class F, class = void>
+struct has_group_sums : std::false_type {};
+template <class F>
+struct has_group_sums<F, std::void_t<decltype(std::declval<const F&>().sum4(0.0, 0.0, 0.0, 0.0))>>
+    : std::true_type {};
+
 template <class F, class = void>
 struct is_exponential : std::false_type {};
 template <class F>
@@ -228,6 +258,23 @@ __device__ __forceinline__ double set_sum(F& f, const double* __restrict__ g,
     acc += call(f, x);
   }
   return acc;
+}
+
+// The rule sums from the sums v[s] over the rule's symmetric sets.  Set 4
+// has a weight in null rule 2 only (rule.cpp's weights()).
+__device__ __forceinline__ void rule_sums(const double (&v)[PAGANI_NSETS],
+                                          const pagani_eval_consts& C,
+                                          double (&rs)[PAGANI_NRULES])
+{
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int r = 0; r < PAGANI_NRULES; ++r) {
+    double acc = C.w[0][r] * v[0];
+#pragma unroll
+    for (int s = 1; s < PAGANI_NSETS; ++s)
+      if (s != 4 || r == 2) acc = __builtin_fma(C.w[s][r], v[s], acc);
+    rs[r] = acc;
+  }
 }
 
 // Rule sums and split axis of one region for a factored separable
@@ -618,6 +665,121 @@ __device__ __forceinline__ bool separable_sums(F& f, const double (&cR)[D], cons
   }
 }
 
+// Rule sums and split axis of one region for an additive integrand with group
+// sums (has_group_sums): a point's value is outer of the centre's joined
+// terms plus the moved axes' changes, and the points of a set are taken in
+// groups of two and four.  The groups are dealt to the `slices` waves that
+// share the batch in turn (uniformly, so a wave's loops hold scalars only);
+// wave 0 also takes sets 0-4, whose axis points give the fourth differences.
+// Without contraction, so every kernel that inlines this forms the same bits.
+// Bound by FP64 issue: 1 105 points at 8D, 10 instructions each.
+template <int D, class F>
+__device__ __forceinline__ bool group_sums(F& f, const double (&cR)[D], const double (&hR)[D],
+                                           const pagani_eval_consts& C, int slices, int wave,
+                                           double (&rs)[PAGANI_NRULES], int& bisect)
+{
+#pragma clang fp contract(off)
+  if (!f.sum_safe(cR, hR)) return false;
+  double T0[D], S0;
+#pragma unroll
+  for (int j = 0; j < D; ++j) {
+    T0[j] = f.term(j, cR[j]);
+    S0 = j ? S0 + T0[j] : T0[0];
+  }
+  auto change = [&](int j, double g) {
+    return f.term(j, __builtin_fma(g, hR[j], cR[j])) - T0[j];
+  };
+  double v[PAGANI_NSETS] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  double d1p[D], d1n[D], d2p[D], d2n[D];  // at x = c - lambda h and c + lambda h
+#pragma unroll
+  for (int j = 0; j < D; ++j) {
+    d1p[j] = change(j, -C.lambda1);
+    d1n[j] = change(j, C.lambda1);
+    d2p[j] = change(j, -C.lambda2);
+    d2n[j] = change(j, C.lambda2);
+  }
+  if (wave == 0) {
+    // sets 0-2 and the fourth differences, Sample.cuh:176-218, and sets 3-4
+    v[0] = f.outer(S0);
+    const double base = v[0] * (2 * (1 - C.ratio));
+    double maxdiff = 0.0;
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      const double fab = f.sum2(S0 + d1p[j], S0 + d1n[j]);
+      const double fcd = f.sum2(S0 + d2p[j], S0 + d2n[j]);
+      v[1] += fab;
+      v[2] += fcd;
+      const double diff = __builtin_fabs(__builtin_fma(C.ratio, fab, base) - fcd);
+      if (diff > maxdiff) {
+        maxdiff = diff;
+        bisect = j;
+      }
+      v[3] += f.sum2(S0 + change(j, -C.lambda3), S0 + change(j, C.lambda3));
+      v[4] += f.sum2(S0 + change(j, -C.lambda4), S0 + change(j, C.lambda4));
+    }
+  }
+  int turn = 0;  // the wave that takes the next group
+  auto mine = [&] {
+    const bool m = turn == wave;
+    turn = turn + 1 == slices ? 0 : turn + 1;
+    return m;
+  };
+  // sets 5-7: (+-lambda1, +-lambda1), (+-lambda1, +-lambda2) and the triples
+#pragma unroll 1
+  for (int j = 0; j < D; ++j) {
+    const double aj = S0 + d1p[j], bj = S0 + d1n[j];
+#pragma unroll 1
+    for (int k = 0; k < D; ++k) {
+      if (k == j) continue;
+      if (mine()) v[6] += f.sum4(aj + d2p[k], bj + d2p[k], aj + d2n[k], bj + d2n[k]);
+      if (k < j) continue;
+      const double q0 = aj + d1p[k], q1 = bj + d1p[k], q2 = aj + d1n[k], q3 = bj + d1n[k];
+      if (mine()) v[5] += f.sum4(q0, q1, q2, q3);
+#pragma unroll 1
+      for (int l = k + 1; l < D; ++l) {
+        if (!mine()) continue;
+        v[7] += f.sum4(q0 + d1p[l], q1 + d1p[l], q2 + d1p[l], q3 + d1p[l]);
+        v[7] += f.sum4(q0 + d1n[l], q1 + d1n[l], q2 + d1n[l], q3 + d1n[l]);
+      }
+    }
+  }
+  // set 8: the 2^D corners.  The low LB axes' combined terms are tabulated
+  // once; each group of 2^LB corners adds the high axes' combination.
+  {
+    constexpr int LB = D < 4 ? D : 4;
+    constexpr int HB = D - LB;
+    double tp[D], tn[D];
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      tp[j] = f.term(j, __builtin_fma(-C.lambda5, hR[j], cR[j]));
+      tn[j] = f.term(j, __builtin_fma(C.lambda5, hR[j], cR[j]));
+    }
+    double lo[1 << LB];
+    lo[0] = tp[0];
+    lo[1] = tn[0];
+#pragma unroll
+    for (int j = 1; j < LB; ++j) {
+#pragma unroll
+      for (int q = 0; q < (1 << j); ++q) {
+        lo[q + (1 << j)] = lo[q] + tn[j];
+        lo[q] = lo[q] + tp[j];
+      }
+    }
+#pragma unroll 1
+    for (int hq = 0; hq < (1 << HB); ++hq) {
+      if (!mine()) continue;
+      double hs = 0.0;
+#pragma unroll
+      for (int j = LB; j < D; ++j) hs += ((hq >> (j - LB)) & 1) ? tn[j] : tp[j];
+#pragma unroll
+      for (int q = 0; q < (1 << LB); q += 4)
+        v[8] += f.sum4(lo[q] + hs, lo[q + 1] + hs, lo[q + 2] + hs, lo[q + 3] + hs);
+    }
+  }
+  rule_sums(v, C, rs);
+  return true;
+}
+
 // Rule sums and split axis of one region for a cosine integrand (slices ==
 // 1).  A point that moves v_j by -g_j h_j on a set A of axes has the angle
 // phi0 - sum_A g_j h_j; the rule takes every sign combination of the g_j,
@@ -725,23 +887,71 @@ struct RegionRow {
       axis = -1;
     }
   }
+  // Axis j's bounds, in place, from what is stored: the lower bound, and the
+  // width's level (level form) or the width.  Returns the width's level.
+  __device__ __forceinline__ int derive(int j, double& lo, double& len, int lev) const
+  {
+    const bool halved = j == axis;
+    if (h0) {
+      lev += halved ? 1 : 0;
+      len = __builtin_ldexp(h0[j], -lev);
+    } else if (halved) {
+      len = len / 2;
+    }
+    if (halved && right) lo = lo + len;
+    return lev;
+  }
   __device__ __forceinline__ void bounds(const double* __restrict__ L,
                                          const double* __restrict__ H, int j, double& lo,
                                          double& len) const
   {
     const std::size_t o = static_cast<std::size_t>(j) * stride + row;
+    int lev = 0;
     lo = L[o];
     if (h0)
-      len = __builtin_ldexp(h0[j], -static_cast<int>(reinterpret_cast<const std::uint16_t*>(H)[o]));
+      lev = reinterpret_cast<const std::uint16_t*>(H)[o];
     else
       len = H[o];
-    if (j == axis) {
-      const double half = len / 2;
-      if (right) lo = lo + half;
-      len = half;
+    derive(j, lo, len, lev);
+  }
+};
+
+// A region's row as stored, read in one go.
+template <int D>
+struct LoadedRow {
+  RegionRow rr;
+  double lo[D], len[D];
+  int lev[D];
+  __device__ __forceinline__ LoadedRow(const double* __restrict__ L, const double* __restrict__ H,
+                                     const std::uint8_t* __restrict__ pdim, std::size_t n,
+                                     std::size_t t, const pagani_eval_consts& C)
+      : rr(pdim, n, t, C.levels ? C.h0 : nullptr)
+  {
+    // one uniform branch around all the loads, so that they are in flight
+    // together
+    if (rr.h0) {
+#pragma unroll
+      for (int j = 0; j < D; ++j) {
+        const std::size_t o = static_cast<std::size_t>(j) * rr.stride + rr.row;
+        lo[j] = L[o];
+        lev[j] = reinterpret_cast<const std::uint16_t*>(H)[o];
+        len[j] = 0.0;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < D; ++j) {
+        const std::size_t o = static_cast<std::size_t>(j) * rr.stride + rr.row;
+        lo[j] = L[o];
+        len[j] = H[o];
+        lev[j] = 0;
+      }
     }
   }
 };
+
+// A product that may be contracted into a sum it is added to where that sum
+// allows contraction (an angle summed over the axes).
+__device__ __forceinline__ double scaled(double x, double a) { return x * a; }
 
 // Region setup, Phases.cuh:323-349: volume, widest axis, and the centre /
 // width of region t in the integrand's frame (user coordinates, moved to the
@@ -754,17 +964,18 @@ __device__ __forceinline__ void region_frame(F& f, const double* __restrict__ L,
                                              double (&cR)[D], double (&hR)[D], double& vol,
                                              int& maxdim)
 {
+#pragma clang fp contract(off)
   const double* lows = C.lows;
   const double* range = C.range;
   double maxr = 0.0;
   vol = 1.0;
   maxdim = 0;
-  const RegionRow rr(pdim, n, t, C.levels ? C.h0 : nullptr);
+  LoadedRow<D> row(L, H, pdim, n, t, C);
 #pragma unroll
   for (int j = 0; j < D; ++j) {
-    double lo, len;
-    rr.bounds(L, H, j, lo, len);
-    const double up = lo + len;
+    row.rr.derive(j, row.lo[j], row.len[j], row.lev[j]);
+    const double lo = row.lo[j];
+    const double up = lo + row.len[j];
     const double r = up - lo;
     vol *= r;
     if (r > maxr) {
@@ -778,10 +989,216 @@ __device__ __forceinline__ void region_frame(F& f, const double* __restrict__ L,
     hR[j] = r * range[j];
     if constexpr (has_origin<F>::value) cR[j] -= f.origin(j);
     if constexpr (has_origin<F>::value && has_axis_scale<F>::value) {
-      cR[j] *= f.axis_scale(j);
-      hR[j] *= f.axis_scale(j);
+      cR[j] = scaled(cR[j], f.axis_scale(j));
+      hR[j] = scaled(hR[j], f.axis_scale(j));
     }
   }
+}
+
+// The LDS tables of a workgroup that evaluates a has_pair_sums integrand on a
+// level-form list: the functor's own table, then the width values of every
+// axis at levels 0 .. kPairLevels<D> - 1.  A list holds a handful of different
+// widths per axis, so these are formed once per workgroup instead of once per
+// region; regions at deeper levels form them in place, to the same bits.
+template <int D>
+constexpr int kPairLevels = 96 / D > 12 ? 96 / D : 12;
+
+template <int D, class F>
+constexpr int pair_table_size()
+{
+  if constexpr (has_pair_sums<F>::value)
+    return F::kTableSize + kPairLevels<D> * D * F::kWidthValues;
+  else
+    return 0;
+}
+
+// region_frame's width of an axis of a region r wide
+template <class F>
+__device__ __forceinline__ double pair_width(F& f, int j, double r, const double* range)
+{
+#pragma clang fp contract(off)
+  double h = r * range[j];
+  if constexpr (has_axis_scale<F>::value) h *= f.axis_scale(j);
+  return h;
+}
+
+// Every thread of the workgroup calls it; a barrier follows before the
+// tables' first use.
+template <int D, class F>
+__device__ __forceinline__ void fill_pair_tables(F& f, const pagani_eval_consts& C, double* tab,
+                                                 int tid, int threads)
+{
+  if constexpr (F::kTableSize > 0) f.fill_table(tab, tid, threads);
+  if constexpr (F::kWidthValues > 0) {
+    for (int e = tid; e < kPairLevels<D> * D; e += threads) {
+      const int lev = e / D, j = e - D * lev;
+      // selects, not an index: the launch arguments stay in scalar registers
+      // (read by lane they are a trip to host memory)
+      double a = 0.0;
+#pragma unroll
+      for (int k = 0; k < D; ++k) {
+        const double r = __builtin_ldexp(C.h0[k], -lev);
+        a = j == k ? f.width_arg(k, pair_width(f, k, r, C.range)) : a;
+      }
+      double w[F::kWidthValues];
+      f.width_values(a, w);
+      double* out = tab + F::kTableSize + e * F::kWidthValues;
+#pragma unroll
+      for (int i = 0; i < F::kWidthValues; ++i) out[i] = w[i];
+    }
+  }
+}
+
+// Rule sums and split axis of region t for an integrand that gives its pair
+// sums, with the region's volume.  A point's value is the centre's value
+// times the changed axes' factors, so a set's sum over its sign combinations
+// factors into the axes' pair sums: the 4 points (+-l1, +-l1) on axes j, k
+// sum to S0 s_j s_k, the 2^D corners to S0 prod_j s5_j.  With masks an
+// unmoved axis contributes u_j = [valid at the centre], and the sum over the
+// sets of m moved axes is the x^m coefficient of prod_j (u_j + x s_j) (set
+// 6: the xy coefficient of prod_j (u_j + x s1_j + y s2_j)).  One pass over
+// the axes, from their bounds to their share of every sum, so no per-axis
+// array is kept; the fourth differences are compared up to the common factor
+// S0 jac.  Without contraction, so every kernel that inlines this forms the
+// same bits.  Returns false, with the region to be evaluated by the generic
+// loop, where the sums would leave the range.
+template <int D, class F>
+__device__ __forceinline__ bool pair_region(F& f, LoadedRow<D>& row, const double* __restrict__ L,
+                                            const double* __restrict__ H, const double* lows,
+                                            const double* range, const pagani_eval_consts& C,
+                                            const double* tab, double (&rs)[PAGANI_NRULES],
+                                            int& bisect, double& vol)
+{
+#pragma clang fp contract(off)
+  constexpr bool kMasked = is_masked<F>::value;
+  constexpr int NW = F::kWidthValues;
+  const RegionRow& rr = row.rr;
+  double(&cj)[D] = row.lo;
+  double(&len)[D] = row.len;
+  const double k0 = 2 * (1 - C.ratio);
+  double maxdiff = 0.0;
+  int axis = -1;
+  vol = 1.0;
+  typename F::Centre centre;
+  std::uint32_t vmask = 0;  // axes invalid at the centre
+  double dv[kMasked ? D : 1];  // the pair sums' part of the fourth differences
+  double acc3 = 0.0, E3 = 1.0, acc4 = 0.0, E4 = 1.0;  // sets 3, 4
+  // the coefficients of sets 1, 2, 5-7 and the lower ones they are built from
+  double e0 = 1.0, e2 = 0.0, e3 = 0.0, g10 = 0.0, g01 = 0.0, g11 = 0.0;
+  double prod = 1.0;  // set 8
+#pragma unroll
+  for (int j = 0; j < D; ++j) {
+    // region_frame's centre and width of axis j
+    const int lev = rr.derive(j, cj[j], len[j], row.lev[j]);
+    const double lo = cj[j], up = lo + len[j], r = up - lo;
+    vol *= r;
+    double c = __builtin_fma(0.5 * (lo + up), range[j], lows[j]);
+    const double h = pair_width(f, j, r, range);
+    c -= f.origin(j);
+    c *= f.axis_scale(j);
+    centre.add(f, j, c, h);
+    double w[NW > 0 ? NW : 1];
+    if constexpr (NW > 0) {
+      // (r == len: the width as the tables have it, whatever the bounds' sum
+      // rounded to)
+      if (tab && lev < kPairLevels<D> && r == len[j]) {
+        const double* ws = tab + F::kTableSize + (lev * D + j) * NW;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) w[i] = ws[i];
+      } else {
+        f.width_values(f.width_arg(j, h), w);
+      }
+    }
+    double s[5];
+    f.pair_sums(j, c, h, w, tab, s);
+    // the fourth difference, Sample.cuh:176-218 (with masks, once it is known
+    // which axes are valid at the centre)
+    if constexpr (kMasked) {
+      dv[j] = __builtin_fma(C.ratio, s[0], -s[1]);
+    } else {
+      const double diff = __builtin_fabs(__builtin_fma(C.ratio, s[0], k0) - s[1]);
+      if (diff > maxdiff) {
+        maxdiff = diff;
+        axis = j;
+      }
+    }
+    if constexpr (kMasked) {
+      const bool in = f.valid(j, c);
+      if (!in) vmask |= 1u << j;
+      const double uj = in ? 1.0 : 0.0;
+      acc3 = __builtin_fma(E3, s[2], acc3 * uj);
+      E3 *= uj;
+      acc4 = __builtin_fma(E4, s[3], acc4 * uj);
+      E4 *= uj;
+      e3 = __builtin_fma(e2, s[0], e3 * uj);
+      e2 = __builtin_fma(g10, s[0], e2 * uj);
+      g11 = __builtin_fma(g01, s[0], __builtin_fma(g10, s[1], g11 * uj));
+      g10 = __builtin_fma(e0, s[0], g10 * uj);
+      g01 = __builtin_fma(e0, s[1], g01 * uj);
+      e0 *= uj;
+    } else {
+      acc3 += s[2];
+      acc4 += s[3];
+      e3 = __builtin_fma(e2, s[0], e3);
+      e2 = __builtin_fma(g10, s[0], e2);
+      g11 = __builtin_fma(g01, s[0], __builtin_fma(g10, s[1], g11));
+      g10 += s[0];
+      g01 += s[1];
+    }
+    prod *= s[4];
+    // axis after axis: interleaved, the axes' temporaries would not fit the
+    // registers of four waves per SIMD
+    if (j + 1 < D)
+      asm volatile("" : "+v"(cj[j + 1 < D ? j + 1 : j]), "+v"(row.lev[j + 1 < D ? j + 1 : j])
+                   : "v"(prod), "v"(e3), "v"(g11), "v"(acc3), "v"(acc4), "v"(maxdiff));
+  }
+  if (!centre.safe(f)) return false;
+  if constexpr (kMasked) {
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      const double diff =
+          __builtin_fabs((vmask ? 0.0 : k0) + ((vmask & ~(1u << j)) ? 0.0 : dv[j]));
+      if (diff > maxdiff) {
+        maxdiff = diff;
+        axis = j;
+      }
+    }
+  }
+  const double S0 = centre.value(f);
+  const double v[PAGANI_NSETS] = {
+      f.value(kMasked && vmask ? 0.0 : S0),
+      f.value(S0 * g10), f.value(S0 * g01), f.value(S0 * acc3), f.value(S0 * acc4),
+      f.value(S0 * e2),  f.value(S0 * g11), f.value(S0 * e3),   f.value(S0 * prod)};
+  rule_sums(v, C, rs);
+  if constexpr (kMasked) {
+    // a masked integrand's factors are bounded only by the box: a region
+    // whose sums left the range takes the generic loop
+    double t = 0.0;
+#pragma unroll
+    for (int r = 0; r < PAGANI_NRULES; ++r) t += __builtin_fabs(rs[r]);
+    if (!__builtin_isfinite(t)) {
+#pragma unroll
+      for (int r = 0; r < PAGANI_NRULES; ++r) rs[r] = 0.0;
+      return false;
+    }
+  }
+  if (axis < 0) {
+    // no fourth difference is positive: the widest axis
+    double maxr = 0.0;
+    axis = 0;
+#pragma unroll 1
+    for (int j = 0; j < D; ++j) {
+      double lo, w;
+      rr.bounds(L, H, j, lo, w);
+      const double r = (lo + w) - lo;
+      if (r > maxr) {
+        maxr = r;
+        axis = j;
+      }
+    }
+  }
+  bisect = axis;
+  return true;
 }
 
 // The tile of workgroup b of a grid of g: workgroups are dealt to the eight
@@ -819,27 +1236,54 @@ __device__ __forceinline__ double point_generator(const pagani_eval_consts& C, i
 // == 1); with more than one, every wave of the workgroup passes one barrier,
 // and only wave 0 returns true (holding the results).  `lows`, `range`,
 // `jac` describe the integration box.
-template <int D, class F, class Real>
+template <int D, class F, class Real, bool Pairs>
 __device__ __forceinline__ bool eval_region_values(
     F& f, const double* __restrict__ L, const double* __restrict__ H,
     const std::uint8_t* __restrict__ pdim, std::size_t n, std::size_t t,
     const double* lows, const double* range, double jac, const pagani_eval_consts& C, int slices,
-    int wave, int lane, double* part, double& avg_out, double& er_out, int& axis_out)
+    int wave, int lane, double* part, LoadedRow<Pairs ? D : 1>* row, const double* tab,
+    double& avg_out, double& er_out, int& axis_out)
 {
-  double cR[D], hR[D];
+#pragma clang fp contract(off)
   double vol;
-  int maxdim;
-  region_frame<D>(f, L, H, pdim, n, t, C, cR, hR, vol, maxdim);
-
   double rs[PAGANI_NRULES] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  int bisect = maxdim;
-
+  int bisect = 0;
   bool done = false;
-  if constexpr (is_cosine<F>::value && has_origin<F>::value && has_axis_scale<F>::value) {
+  double cR[D], hR[D];
+  if constexpr (Pairs)
+    done = pair_region<D, F>(f, *row, L, H, lows, range, C, tab, rs, bisect, vol);
+  if (!done) {
+    // nothing of the pair sums is worth keeping for the rare region that
+    // takes the generic loop after them: the compiler must not see that the
+    // two share values
+    if constexpr (Pairs) asm volatile("" : "+v"(t));
+    region_frame<D>(f, L, H, pdim, n, t, C, cR, hR, vol, bisect);
+  }
+  if constexpr (has_group_sums<F>::value) {
+    done = group_sums<D, F>(f, cR, hR, C, slices, wave, rs, bisect);
+  } else if constexpr (has_pair_sums<F>::value) {
+    // a region out of the pair sums' range, and several waves: the generic loop
+  } else if constexpr (is_cosine<F>::value && has_origin<F>::value && has_axis_scale<F>::value) {
     if (slices == 1) done = cosine_sums<D, F, Real>(f, cR, hR, jac, C, rs, bisect);
   } else if constexpr (is_separable<F>::value) {
     if (slices == 1) done = separable_sums<D, F>(f, cR, hR, jac, C, rs, bisect);
   }
+  // Wave 0 adds the waves' partial sums (true); the others are through.
+  auto combine = [&] {
+    if (wave > 0) {
+#pragma unroll
+      for (int r = 0; r < PAGANI_NRULES; ++r)
+        part[((wave - 1) * PAGANI_NRULES + r) * 64 + lane] = rs[r];
+    }
+    __syncthreads();
+    if (wave > 0) return false;
+    for (int w = 1; w < slices; ++w) {
+#pragma unroll
+      for (int r = 0; r < PAGANI_NRULES; ++r)
+        rs[r] += part[((w - 1) * PAGANI_NRULES + r) * 64 + lane];
+    }
+    return true;
+  };
   if (!done) {
     if (wave == 0) {
       // Centre and the +-lambda1, +-lambda2 axis points (sets 0-2), whose
@@ -865,14 +1309,14 @@ __device__ __forceinline__ bool eval_region_values(
         const double fd = moved(j, -C.lambda2);
         s1 += fa + fb;
         s2 += fc + fd;
-        const double diff = __builtin_fabs(
-            base + C.ratio * (fa * jac + fb * jac) - (fc * jac + fd * jac));
+        const double ab = __builtin_fma(fa, jac, fb * jac), cd = __builtin_fma(fc, jac, fd * jac);
+        const double diff = __builtin_fabs(__builtin_fma(C.ratio, ab, base) - cd);
         if (diff > maxdiff) {
           maxdiff = diff;
           bisect = j;
         }
       };
-      if constexpr (heavy_outer<F>::value) {
+      if constexpr (heavy_outer<F>::value || Pairs) {
         // a long integrand: one copy of the four evaluations, the axis
         // chosen by selects
 #pragma unroll 1
@@ -883,7 +1327,7 @@ __device__ __forceinline__ bool eval_region_values(
       }
 #pragma unroll
       for (int r = 0; r < PAGANI_NRULES; ++r)
-        rs[r] = C.w[0][r] * f0 + C.w[1][r] * s1 + C.w[2][r] * s2;
+        rs[r] = __builtin_fma(C.w[2][r], s2, __builtin_fma(C.w[1][r], s1, C.w[0][r] * f0));
     }
 
     // Sets 3..8 from the generator table, this wave's slice of the points.
@@ -902,24 +1346,12 @@ __device__ __forceinline__ bool eval_region_values(
           rs[r] = __builtin_fma(C.w[s][r], acc, rs[r]);
       }
     }
-
-    if (slices > 1) {
-      if (wave > 0) {
-#pragma unroll
-        for (int r = 0; r < PAGANI_NRULES; ++r)
-          part[((wave - 1) * PAGANI_NRULES + r) * 64 + lane] = rs[r];
-      }
-      __syncthreads();
-      if (wave == 0) {
-        for (int w = 1; w < slices; ++w) {
-#pragma unroll
-          for (int r = 0; r < PAGANI_NRULES; ++r)
-            rs[r] += part[((w - 1) * PAGANI_NRULES + r) * 64 + lane];
-        }
-      }
-      if (wave > 0) return false;
-    }
+    if constexpr (!has_group_sums<F>::value)
+      if (slices > 1 && !combine()) return false;
   }
+  // lanes that formed their share either way meet at one barrier
+  if constexpr (has_group_sums<F>::value)
+    if (slices > 1 && !combine()) return false;
 
   // Null-rule error estimate, Sample.cuh:261-289.
   double s[PAGANI_NRULES];
@@ -928,9 +1360,16 @@ __device__ __forceinline__ bool eval_region_values(
   double e1 = 0.0, e2 = 0.0, e3 = 0.0;
 #pragma unroll
   for (int k = 0; k < PAGANI_NSETS; ++k) {
-    e1 = __builtin_fmax(e1, __builtin_fabs(s[2] + C.scale[k][1] * s[1]) * C.norm[k][1]);
-    e2 = __builtin_fmax(e2, __builtin_fabs(s[3] + C.scale[k][2] * s[2]) * C.norm[k][2]);
-    e3 = __builtin_fmax(e3, __builtin_fabs(s[4] + C.scale[k][3] * s[3]) * C.norm[k][3]);
+    // sets 5-8 share null rule 1's combination (their weights in rules 1 and
+    // 2 are opposite) and sets 7-8 null rule 3's: one of each is enough
+    if (k <= 5)
+      e1 = __builtin_fmax(
+          e1, __builtin_fabs(__builtin_fma(C.scale[k][1], s[1], s[2])) * C.norm[k][1]);
+    e2 = __builtin_fmax(
+        e2, __builtin_fabs(__builtin_fma(C.scale[k][2], s[2], s[3])) * C.norm[k][2]);
+    if (k <= 7)
+      e3 = __builtin_fmax(
+          e3, __builtin_fabs(__builtin_fma(C.scale[k][3], s[3], s[4])) * C.norm[k][3]);
   }
   avg_out = vol * s[0];
   er_out = vol * ((5.0 * e1 <= e2 && 5.0 * e2 <= e3)
@@ -941,18 +1380,18 @@ __device__ __forceinline__ bool eval_region_values(
 }
 
 // eval_region_values, stored: region t's estimate, error and split axis.
-template <int D, class F, class Real>
+template <int D, class F, class Real, bool Pairs>
 __device__ __forceinline__ void eval_regions_wave(
     F& f, const double* __restrict__ L, const double* __restrict__ H,
     const std::uint8_t* __restrict__ pdim, std::size_t n, std::size_t t, bool live,
     const double* lows, const double* range, double jac, const pagani_eval_consts& C, int slices,
-    int wave, int lane, double* part, double* __restrict__ est, double* __restrict__ err,
-    std::uint8_t* __restrict__ dim)
+    int wave, int lane, double* part, LoadedRow<Pairs ? D : 1>* row, const double* tab,
+    double* __restrict__ est, double* __restrict__ err, std::uint8_t* __restrict__ dim)
 {
   double avg, er;
   int axis;
-  if (!eval_region_values<D, F, Real>(f, L, H, pdim, n, t, lows, range, jac, C, slices, wave,
-                                      lane, part, avg, er, axis))
+  if (!eval_region_values<D, F, Real, Pairs>(f, L, H, pdim, n, t, lows, range, jac, C, slices, wave,
+                                      lane, part, row, tab, avg, er, axis))
     return;
   if (live) {
     est[t] = avg;
@@ -963,18 +1402,68 @@ __device__ __forceinline__ void eval_regions_wave(
 
 }  // namespace detail
 
-// Kernel: workgroup b evaluates a batch of 64 regions of an n-region SoA
-// list (flat: [64 b, 64 b + 64); split form when P is given: the children
-// of parents [32 b, 32 b + 32)) with S = slices waves sharing the batch's
-// points.  For a
-// host-driven launch `it` is NULL and n, the pool (L0, H0) and S = C.slices
-// come from the arguments.  In the device-resident loop they come from *it
-// (nothing at all if !it->run), and the launch is sized for the round's
-// largest list: workgroups past n return at once, and waves past the
-// iteration's slice count only keep the barrier company.  Both forms run
-// this one kernel, so a given n and slice count give the same bits either
-// way.  Dynamic LDS: (waves per workgroup - 1)*5*64 doubles.
-template <int D, class F, class Real>
+// What a launch evaluates: for a host-driven launch `it` is NULL and n, the
+// pool (L0, H0, P0) and the slice count come from the arguments; in the
+// device-resident loop they come from *it (nothing at all if !it->run), and
+// the launch is sized for the round's largest list, so workgroups past n
+// return at once.
+struct LaunchList {
+  std::size_t n;
+  const double *L, *H;
+  const std::uint8_t* P;
+  int slices;
+  __device__ __forceinline__ bool resolve(const pagani_dev_iter* it, std::size_t n_arg,
+                                          const double* L0, const double* H0, const double* L1,
+                                          const double* H1, const std::uint8_t* P0,
+                                          const std::uint8_t* P1, int s)
+  {
+    n = n_arg;
+    L = L0;
+    H = H0;
+    P = P0;
+    slices = s;
+    if (it) {
+      if (!it->run) return false;
+      n = it->n;
+      if (it->cur) {
+        L = L1;
+        H = H1;
+        P = P1;
+      }
+      if (!it->split) P = nullptr;
+      slices = static_cast<int>(it->slices);
+    }
+    return true;
+  }
+  // The region lane `lane` of tile `tile` takes.  A flat list gives tile b
+  // the regions 64 b + lane.  A split list (n = 2m children, child t of
+  // parent t mod m) gives it both children of the parents 32 b .. 32 b + 31:
+  // lanes l and l + 32 read the same parent row in one load instruction, so
+  // each row leaves HBM once, and the writes are two runs of 32 consecutive
+  // regions.
+  __device__ __forceinline__ void region(std::size_t tile, int lane, std::size_t& t,
+                                         bool& live) const
+  {
+    if (P) {
+      const std::size_t m = n / 2;
+      const std::size_t p0 = tile * 32 + (lane & 31);
+      live = p0 < m;
+      t = (live ? p0 : m - 1) + (lane >= 32 ? m : 0);
+    } else {
+      const std::size_t t0 = tile * 64 + lane;
+      live = t0 < n;
+      t = live ? t0 : n - 1;
+    }
+  }
+};
+
+// Kernel: workgroup b evaluates a tile of 64 regions of an n-region SoA list
+// with S = slices waves sharing the tile's points; waves past the
+// iteration's slice count only keep the barrier company.  Host-driven and
+// device-loop launches run this one kernel, so a given n and slice count
+// give the same bits either way.  Dynamic LDS: (waves per workgroup -
+// 1)*5*64 doubles.  Pairs: the pair sums without tables (slices == 1).
+template <int D, class F, class Real, bool Pairs>
 __global__ void __launch_bounds__(64 * PAGANI_MAX_SLICES)
     eval_kernel(F f, const pagani_dev_iter* __restrict__ it, std::size_t n_arg,
                 const double* __restrict__ L0, const double* __restrict__ H0,
@@ -984,53 +1473,84 @@ __global__ void __launch_bounds__(64 * PAGANI_MAX_SLICES)
                 std::uint8_t* __restrict__ dim, const pagani_eval_consts C)
 {
   extern __shared__ double part[];
-  std::size_t n = n_arg;
-  const double* L = L0;
-  const double* H = H0;
-  const std::uint8_t* P = P0;
-  int slices = C.slices;
-  if (it) {
-    if (!it->run) return;
-    n = it->n;
-    if (it->cur) {
-      L = L1;
-      H = H1;
-      P = P1;
-    }
-    if (!it->split) P = nullptr;
-    slices = static_cast<int>(it->slices);
-  }
+  LaunchList list;
+  if (!list.resolve(it, n_arg, L0, H0, L1, H1, P0, P1, C.slices)) return;
   // the list's tiles of 64 regions; workgroups past them return at once
-  const std::size_t tiles = (n + 63) / 64;
+  const std::size_t tiles = (list.n + 63) / 64;
   if (blockIdx.x >= tiles) return;
   const std::size_t tile = detail::xcd_tile(blockIdx.x, static_cast<unsigned>(tiles));
   const int lane = threadIdx.x & 63;
   // wave index is uniform across the wave: keep it (and everything derived
   // from it, the slice bounds and the point loop) in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  if (wave >= slices) {
-    if (slices > 1) __syncthreads();
+  if (wave >= list.slices) {
+    if (list.slices > 1) __syncthreads();
     return;
   }
-  // A flat list gives tile b the regions 64 b + lane.  A split list (n = 2m
-  // children, child t of parent t mod m) gives it both children of the
-  // parents 32 b .. 32 b + 31: lanes l and l + 32 read the same parent row
-  // in one load instruction, so each row leaves HBM once, and the writes are
-  // two runs of 32 consecutive regions.
   std::size_t t;
   bool live;
-  if (P) {
-    const std::size_t m = n / 2;
-    const std::size_t p0 = tile * 32 + (lane & 31);
-    live = p0 < m;
-    t = (live ? p0 : m - 1) + (lane >= 32 ? m : 0);
+  list.region(tile, lane, t, live);
+  if constexpr (Pairs) {
+    detail::LoadedRow<D> row(list.L, list.H, list.P, list.n, t, C);
+    detail::eval_regions_wave<D, F, Real, true>(f, list.L, list.H, list.P, list.n, t, live, C.lows,
+                                                C.range, C.jac, C, 1, 0, lane, nullptr, &row,
+                                                nullptr, est, err, dim);
   } else {
-    const std::size_t t0 = tile * 64 + lane;
-    live = t0 < n;
-    t = live ? t0 : n - 1;
+    detail::eval_regions_wave<D, F, Real, false>(f, list.L, list.H, list.P, list.n, t, live,
+                                                 C.lows, C.range, C.jac, C, list.slices, wave,
+                                                 lane, part, nullptr, nullptr, est, err, dim);
   }
-  detail::eval_regions_wave<D, F, Real>(f, L, H, P, n, t, live, C.lows, C.range, C.jac, C,
-                                        slices, wave, lane, part, est, err, dim);
+}
+
+// Waves of pair_kernel's workgroups: each takes a tile of its own, and they
+// share the LDS tables.  Eight, so that forming the tables is a few per cent
+// of the evaluation (8D Gaussian: 47 ms per headline integral against 51 with
+// four); a masked integrand keeps its axes' differences and needs the
+// registers of three waves per SIMD, so workgroups of four.
+template <class F>
+constexpr int kPairWaves = detail::is_masked<F>::value ? 4 : 8;
+template <class F>
+constexpr int kPairPerSimd = detail::is_masked<F>::value ? 3 : 4;
+// tiles from which a level-form list takes pair_kernel
+constexpr std::size_t kPairLong = 4096;
+
+// Kernel: the evaluation of a has_pair_sums integrand on a level-form list at
+// one wave per tile of 64 regions (slices == 1), with its tables.
+template <int D, class F>
+__global__ void __launch_bounds__(64 * kPairWaves<F>, kPairPerSimd<F>)
+    pair_kernel(F f, const pagani_dev_iter* __restrict__ it, std::size_t n_arg,
+                const double* __restrict__ L0, const double* __restrict__ H0,
+                const double* __restrict__ L1, const double* __restrict__ H1,
+                const std::uint8_t* __restrict__ P0, const std::uint8_t* __restrict__ P1,
+                double* __restrict__ est, double* __restrict__ err,
+                std::uint8_t* __restrict__ dim, const pagani_eval_consts C)
+{
+  constexpr int kTab = detail::pair_table_size<D, F>();
+  __shared__ double tab[kTab > 0 ? kTab : 1];
+  LaunchList list;
+  if (!list.resolve(it, n_arg, L0, H0, L1, H1, P0, P1, 1)) return;
+  const unsigned waves = blockDim.x >> 6;
+  const std::size_t tiles = (list.n + 63) / 64;
+  const std::size_t groups = (tiles + waves - 1) / waves;
+  if (blockIdx.x >= groups) return;
+  const std::size_t tile =
+      detail::xcd_tile(blockIdx.x, static_cast<unsigned>(groups)) * waves +
+      static_cast<std::size_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
+  const int lane = threadIdx.x & 63;
+  std::size_t t;
+  bool live;
+  list.region(tile, lane, t, live);  // a tile past the list: its last region, not stored
+  // the region's row is on its way while the tables are formed
+  detail::LoadedRow<D> row(list.L, list.H, list.P, list.n, t, C);
+  if constexpr (kTab > 0) {
+    const int threads = static_cast<int>(blockDim.x);
+    detail::fill_pair_tables<D>(f, C, tab, threadIdx.x, threads);
+    __syncthreads();
+  }
+  if (tile >= tiles) return;
+  detail::eval_regions_wave<D, F, double, true>(f, list.L, list.H, list.P, list.n, t, live, C.lows,
+                                                C.range, C.jac, C, 1, 0, lane, nullptr, &row, tab,
+                                                est, err, dim);
 }
 
 // The debug recorder's point dump: thread i writes the value at rule point
@@ -1071,15 +1591,31 @@ int eval_regions(const F& f, const pagani_eval_args* args)
   // loop's counts for its launches)
   const int waves = args->consts.slices;
   if (waves < 1 || waves > PAGANI_MAX_SLICES) return PAGANI_EBADARG;
-  const std::size_t blocks = (args->n + 63) / 64;
-  const std::size_t lds =
-      waves > 1 ? static_cast<std::size_t>(waves - 1) * PAGANI_NRULES * 64 * sizeof(double) : 0;
-  hipLaunchKernelGGL((eval_kernel<D, F, Real>), dim3(static_cast<unsigned>(blocks)),
-                     dim3(64 * waves), lds, static_cast<hipStream_t>(args->stream), f, args->dev,
-                     args->n, args->L, args->H, args->dev ? args->L2 : args->L,
-                     args->dev ? args->H2 : args->H, args->pdim,
-                     args->dev ? args->pdim2 : args->pdim, args->est, args->err, args->dim,
-                     args->consts);
+  const std::size_t tiles = (args->n + 63) / 64;
+  auto launch = [&](auto kernel, std::size_t blocks, int threads, std::size_t lds) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(threads), lds,
+                       static_cast<hipStream_t>(args->stream), f, args->dev, args->n, args->L,
+                       args->H, args->dev ? args->L2 : args->L, args->dev ? args->H2 : args->H,
+                       args->pdim, args->dev ? args->pdim2 : args->pdim, args->est, args->err,
+                       args->dim, args->consts);
+  };
+  bool pairs = false;
+  if constexpr (detail::has_pair_sums<F>::value && std::is_same_v<Real, double>) {
+    pairs = waves == 1;
+    // Tables where they pay: long lists in level form.  Forming them is 2 us
+    // before a workgroup's first region, and a list that leaves waves idle
+    // waits for it; a list with its widths as doubles has none.
+    bool tables = false;
+    if constexpr (detail::pair_table_size<D, F>() > 0) {
+      tables = pairs && args->consts.levels && tiles >= kPairLong;
+      const int pw = kPairWaves<F>;
+      if (tables) launch(pair_kernel<D, F>, (tiles + pw - 1) / pw, 64 * pw, 0);
+    }
+    if (pairs && !tables) launch(eval_kernel<D, F, Real, true>, tiles, 64, 0);
+  }
+  if (!pairs)
+    launch(eval_kernel<D, F, Real, false>, tiles, 64 * waves,
+           static_cast<std::size_t>(waves - 1) * PAGANI_NRULES * 64 * sizeof(double));
   if (args->fevals && !args->dev) {
     const std::size_t threads = args->n * static_cast<std::size_t>(args->consts.feval);
     hipLaunchKernelGGL((point_values_kernel<D, F, Real>), dim3(static_cast<unsigned>((threads + 255) / 256)),

@@ -69,7 +69,153 @@ __device__ __forceinline__ double fabs_(double x) { return __builtin_fabs(x); }
 __device__ __forceinline__ float fabs_(float x) { return __builtin_fabsf(x); }
 __device__ __forceinline__ double fmax_(double x, double y) { return __builtin_fmax(x, y); }
 __device__ __forceinline__ float fmax_(float x, float y) { return __builtin_fmaxf(x, y); }
+// written out where a sum is contracted, so that every kernel an integrand
+// is inlined into forms the same bits
+__device__ __forceinline__ double fma_(double x, double y, double z) { return __builtin_fma(x, y, z); }
+__device__ __forceinline__ float fma_(float x, float y, float z) { return __builtin_fmaf(x, y, z); }
 }  // namespace math
+
+// The rule's generator magnitudes lambda1..lambda5 (rule.cpp's kLam): the
+// points of one axis are c -+ lambda_i h.
+constexpr double kLambda[5] = {.4779536579022695061928604197171830064732,
+                               .2030285873691198677998034402373279133258,
+                               .4476273546261781288207704806530998539285, .125,
+                               .3430378987808781457001426145164678603407};
+constexpr double lambda2(int i) { return kLambda[i] * kLambda[i]; }
+
+// Truncated Taylor series and the rule's magnitudes, for the pair sums of the
+// factored integrands (eval_kernel.hpp, has_pair_sums).
+namespace series {
+constexpr double factorial(int n)
+{
+  double f = 1.0;
+  for (int k = 2; k <= n; ++k) f *= k;
+  return f;
+}
+// The degree N in z of sum_k z^k / (Step k + Off)! whose first term left out
+// is at most 2^-56 for 0 <= z <= zmax (the sums here are at least 1).
+constexpr int degree(double zmax, int Step, int Off = 0)
+{
+  double p = zmax;
+  for (int n = 0;; ++n, p *= zmax)
+    if (p <= 0x1p-56 * factorial(Step * (n + 1) + Off)) return n;
+}
+// sum_{k <= N} z^k / (Step k + Off)!
+template <int N, int Step, int Off>
+__device__ __forceinline__ double sum(double z)
+{
+#pragma clang fp contract(off)
+  double p = 1.0 / factorial(Step * N + Off);
+#pragma unroll
+  for (int k = N - 1; k >= 0; --k) p = __builtin_fma(p, z, 1.0 / factorial(Step * k + Off));
+  return p;
+}
+// fn(std::integral_constant<int, i>) for the rule's five magnitudes
+template <class Fn>
+__device__ __forceinline__ void for_lambda(Fn&& fn)
+{
+  fn(std::integral_constant<int, 0>{});
+  fn(std::integral_constant<int, 1>{});
+  fn(std::integral_constant<int, 2>{});
+  fn(std::integral_constant<int, 3>{});
+  fn(std::integral_constant<int, 4>{});
+}
+}  // namespace series
+
+// The largest centre sum s0 for which an exponential family evaluates a
+// region as products: e^s0 and e^-s0 stay normal with room to spare (FP64
+// 2^+-1022 is e^+-708; FP32 2^+-126 is e^+-87).
+template <class Real>
+constexpr double kFactorRange = sizeof(Real) == 8 ? 650.0 : 80.0;
+
+namespace math {
+// e^x (x <= 709) for the product forms of the exponential families: at
+// the integrand's precision where it holds the value (FP32: |x| <= 80),
+// else in FP64, so that an FP32 integrand's centre values and factors stay
+// normal over the FP64 range of the products.
+__device__ __forceinline__ double exp_factor(double x, double) { return exp_bounded(x); }
+
+// 1 / x for finite, normal x: the hardware reciprocal refined by two
+// Newton steps (each doubles the correct bits: r' = r + r (1 - x r)).
+__device__ __forceinline__ double recip(double x)
+{
+  double r = __builtin_amdgcn_rcp(x);
+  double e = __builtin_fma(-x, r, 1.0);
+  r = __builtin_fma(r, e, r);
+  e = __builtin_fma(-x, r, 1.0);
+  return __builtin_fma(r, e, r);
+}
+__device__ __forceinline__ double exp_factor(double x, float)
+{
+  return __builtin_fabs(x) <= 80.0 ? static_cast<double>(::expf(static_cast<float>(x)))
+                                   : exp_bounded(x);
+}
+}  // namespace math
+
+// 2 cosh(l_i n/2) and 2 l_i sinh(l_i n/2) for the rule's five magnitudes and
+// n < kCoshSteps, [(5 n + i) 2], formed by the compiler: the powers of
+// e^(+-l_i/2) in double-double arithmetic (two-sum, and Dekker's product).
+constexpr int kCoshSteps = 201, kCoshLds = 51;
+struct CoshTable {
+  double v[kCoshSteps * 10];
+};
+namespace dd {
+struct Num {
+  double hi, lo;
+};
+constexpr Num norm(double a, double b)
+{
+  const double s = a + b, t = s - a;
+  return {s, (a - (s - t)) + (b - t)};
+}
+constexpr Num add(Num a, Num b)
+{
+  const Num s = norm(a.hi, b.hi);
+  return norm(s.hi, s.lo + a.lo + b.lo);
+}
+constexpr Num mul(Num a, Num b)
+{
+  constexpr double k = 134217729.0;  // 2^27 + 1
+  const double ta = k * a.hi, ah = ta - (ta - a.hi), al = a.hi - ah;
+  const double tb = k * b.hi, bh = tb - (tb - b.hi), bl = b.hi - bh;
+  const double p = a.hi * b.hi;
+  const double e = ((ah * bh - p) + ah * bl + al * bh) + al * bl;
+  return norm(p, e + (a.hi * b.lo + a.lo * b.hi));
+}
+// e^x, |x| < 1/4: the Taylor series by Horner's rule, 1 + x/1 (1 + x/2 (...));
+// the quotients x/k corrected by one residual
+constexpr Num exp(double x)
+{
+  Num s{1.0, 0.0};
+  for (int k = 26; k >= 1; --k) {
+    const double q = x / k;
+    const Num r = mul({q, 0.0}, {static_cast<double>(k), 0.0});
+    s = add({1.0, 0.0}, mul(s, {q, ((x - r.hi) - r.lo) / k}));
+  }
+  return s;
+}
+}  // namespace dd
+constexpr CoshTable make_cosh_table()
+{
+  CoshTable t{};
+  for (int i = 0; i < 5; ++i) {
+    const dd::Num up = dd::exp(.5 * kLambda[i]), down = dd::exp(-.5 * kLambda[i]);
+    dd::Num p{1.0, 0.0}, q{1.0, 0.0};
+    for (int n = 0; n < kCoshSteps; ++n) {
+      t.v[2 * (5 * n + i)] = dd::add(p, q).hi;
+      t.v[2 * (5 * n + i) + 1] = dd::mul(dd::add(p, {-q.hi, -q.lo}), {kLambda[i], 0.0}).hi;
+      p = dd::mul(p, up);
+      q = dd::mul(q, down);
+    }
+  }
+  return t;
+}
+static __device__ const CoshTable kCoshTable = make_cosh_table();
+
+// Marks a member as present for FP64 integrands only (an FP32 integrand
+// keeps its FP32 functions).
+template <class Real>
+using if_double = std::enable_if_t<std::is_same_v<Real, double>, int>;
 
 // cos(2 pi u_0 + sum a_i x_i)
 template <class Real, int D>
@@ -138,9 +284,51 @@ struct ProductPeak {
     const Real v[D] = {static_cast<Real>(vs)...};
     Real den = 1;
 #pragma unroll
-    for (int i = 0; i < D; ++i) den *= Real(1) + v[i] * v[i];
+    for (int i = 0; i < D; ++i) den *= math::fma_(v[i], v[i], Real(1));
     return static_cast<Real>(k2) / den;
   }
+  // With A = 1 + v^2, p = 1 + (v + l h)^2 and q = 1 + (v - l h)^2 the pair's
+  // factors are A/p and A/q, their sum A (p + q) / (p q).  The five
+  // reciprocals of an axis come from one (the product of the five p q, then
+  // unwound), so an axis has one division where the factors one by one have
+  // twenty.  |v|, |h| <= 1e7 keeps that product, and the centre's prod_j A,
+  // below 1e150.
+  struct Centre {
+    double den = 1.0, big = 0.0;
+    __device__ void add(const ProductPeak&, int, double c, double h)
+    {
+      den *= __builtin_fma(c, c, 1.0);
+      big = __builtin_fmax(big, __builtin_fmax(__builtin_fabs(c), __builtin_fabs(h)));
+    }
+    __device__ bool safe(const ProductPeak&) const { return big <= 1e7; }
+    __device__ double value(const ProductPeak&) const { return 1.0 / den; }
+  };
+  static constexpr int kWidthValues = 0, kTableSize = 0;
+  template <class R = Real, if_double<R> = 0>
+  __device__ void pair_sums(int, double v, double h, const double*, const double*,
+                            double (&s)[5]) const
+  {
+#pragma clang fp contract(off)
+    const double A = __builtin_fma(v, v, 1.0);
+    double pq[5], left[5];  // the products p q, and the product of those before
+    double run = 1.0;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      const double vp = __builtin_fma(kLambda[i], h, v), vm = __builtin_fma(-kLambda[i], h, v);
+      const double p = __builtin_fma(vp, vp, 1.0), q = __builtin_fma(vm, vm, 1.0);
+      s[i] = A * (p + q);
+      pq[i] = p * q;
+      left[i] = run;
+      run *= pq[i];
+    }
+    double r = math::recip(run);
+#pragma unroll
+    for (int i = 4; i >= 0; --i) {
+      s[i] *= r * left[i];
+      r *= pq[i];
+    }
+  }
+  __device__ double value(double p) const { return outer(p); }
   static constexpr bool multiplicative = true;
   static constexpr bool linear_outer = true;
   __device__ double term(int, double v) const { return 1.0 / (1.0 + v * v); }
@@ -184,37 +372,56 @@ struct CornerPeak {
   {
     return static_cast<double>(power(static_cast<Real>(1.0 + s)));
   }
+  // outer summed over two and over four points, FP64: the reciprocals of the
+  // bases come from one, that of their product, and a power takes log2(d)
+  // products, so a point costs 10 instructions where a division and d
+  // products cost 27.  sum_safe bounds a region's bases away from zero and
+  // infinity, so the products of four stay in range (every offset of a rule
+  // point is below half the width).
+  template <int N>
+  static __device__ double power_of(double r)
+  {
+    if constexpr (N == 1)
+      return r;
+    else if constexpr (N % 2)
+      return power_of<N - 1>(r) * r;
+    else {
+      const double t = power_of<N / 2>(r);
+      return t * t;
+    }
+  }
+  template <class R = Real, if_double<R> = 0>
+  __device__ bool sum_safe(const double (&c)[D], const double (&h)[D]) const
+  {
+    double s = 1.0, w = 0.0;
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+      s += c[j];
+      w += __builtin_fabs(h[j]);
+    }
+    w *= .5;
+    return s - w >= 1e-30 && s + w <= 1e30;
+  }
+  template <class R = Real, if_double<R> = 0>
+  __device__ double sum2(double s0, double s1) const
+  {
+#pragma clang fp contract(off)
+    const double a = 1.0 + s0, b = 1.0 + s1;
+    const double r = math::recip(a * b);
+    return power_of<D + 1>(b * r) + power_of<D + 1>(a * r);
+  }
+  template <class R = Real, if_double<R> = 0>
+  __device__ double sum4(double s0, double s1, double s2, double s3) const
+  {
+#pragma clang fp contract(off)
+    const double a = 1.0 + s0, b = 1.0 + s1, c = 1.0 + s2, d = 1.0 + s3;
+    const double ab = a * b, cd = c * d;
+    const double r = math::recip(ab * cd);
+    const double rab = r * cd, rcd = r * ab;
+    return (power_of<D + 1>(rab * b) + power_of<D + 1>(rab * a)) +
+           (power_of<D + 1>(rcd * d) + power_of<D + 1>(rcd * c));
+  }
 };
-
-// The largest centre sum s0 for which an exponential family evaluates a
-// region as products: e^s0 and e^-s0 stay normal with room to spare (FP64
-// 2^+-1022 is e^+-708; FP32 2^+-126 is e^+-87).
-template <class Real>
-constexpr double kFactorRange = sizeof(Real) == 8 ? 650.0 : 80.0;
-
-namespace math {
-// e^x (x <= 709) for the product forms of the exponential families: at
-// the integrand's precision where it holds the value (FP32: |x| <= 80),
-// else in FP64, so that an FP32 integrand's centre values and factors stay
-// normal over the FP64 range of the products.
-__device__ __forceinline__ double exp_factor(double x, double) { return exp_bounded(x); }
-
-// 1 / x for finite, normal x: the hardware reciprocal refined by two
-// Newton steps (each doubles the correct bits: r' = r + r (1 - x r)).
-__device__ __forceinline__ double recip(double x)
-{
-  double r = __builtin_amdgcn_rcp(x);
-  double e = __builtin_fma(-x, r, 1.0);
-  r = __builtin_fma(r, e, r);
-  e = __builtin_fma(-x, r, 1.0);
-  return __builtin_fma(r, e, r);
-}
-__device__ __forceinline__ double exp_factor(double x, float)
-{
-  return __builtin_fabs(x) <= 80.0 ? static_cast<double>(::expf(static_cast<float>(x)))
-                                   : exp_bounded(x);
-}
-}  // namespace math
 
 // exp(-sum a_i^2 (x_i - u_i)^2)
 template <class Real, int D>
@@ -246,7 +453,7 @@ struct Gaussian {
     const Real v[D] = {static_cast<Real>(vs)...};
     Real s = v[0] * v[0];
 #pragma unroll
-    for (int i = 1; i < D; ++i) s += v[i] * v[i];  // one FMA per axis (contracted)
+    for (int i = 1; i < D; ++i) s = math::fma_(v[i], v[i], s);
     return math::exp_neg(-s);
   }
   // additively separable in v: f = outer(sum_j term(j, v_j)); the terms
@@ -265,6 +472,77 @@ struct Gaussian {
   __device__ double factor(double d) const { return math::exp_factor(-d, Real()); }
   __device__ double centre_value(double s0) const { return math::exp_factor(-s0, Real()); }
   __device__ bool factor_safe(double s0) const { return s0 <= kFactorRange<double>; }
+  // e^(v^2 - (v - l h)^2) + e^(v^2 - (v + l h)^2) = e^(-(l h)^2) 2 cosh(l y)
+  // with y = 2 v h.  The first factor is a function of the width alone.  For
+  // the second |y| = n/2 + r, |r| <= 1/4: cosh and sinh of l n/2 from a
+  // table, those of l r from short series, so the pair costs 14
+  // instructions where its two exponentials cost 38.  |y| > 100 takes the
+  // exponentials.
+  struct Centre {
+    double sum = 0.0;
+    __device__ void add(const Gaussian&, int, double c, double) { sum = __builtin_fma(c, c, sum); }
+    __device__ bool safe(const Gaussian& f) const { return f.factor_safe(sum); }
+    __device__ double value(const Gaussian&) const { return math::exp_bounded(-sum); }
+  };
+  static constexpr int kWidthValues = 5, kTableSize = kCoshLds * 10;
+  __device__ double width_arg(int, double h) const { return h; }
+  __device__ void width_values(double h, double (&w)[5]) const
+  {
+#pragma clang fp contract(off)
+    const double X = h * h;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) w[i] = math::exp_bounded(-(lambda2(i) * X));
+  }
+  __device__ static void fill_table(double* tab, int tid, int threads)
+  {
+    for (int e = tid; e < kTableSize / 2; e += threads) {
+      const double c = kCoshTable.v[2 * e], s = kCoshTable.v[2 * e + 1];
+      tab[2 * e] = c;
+      tab[2 * e + 1] = s;
+    }
+  }
+  template <class R = Real, if_double<R> = 0>
+  __device__ void pair_sums(int, double v, double h, const double* w, const double* tab,
+                            double (&s)[5]) const
+  {
+#pragma clang fp contract(off)
+    const double y = __builtin_fabs((v + v) * h);
+    if (y <= .5 * (kCoshSteps - 1)) {
+      constexpr double kShift = 0x1.8p+52;
+      const double t = __builtin_fma(y, 2.0, kShift);
+      const int n = static_cast<int>(__builtin_bit_cast(unsigned long long, t));
+      const double r = __builtin_fma(-.5, t - kShift, y), R2 = r * r;
+      // the table's first rows are in LDS, all of it in memory
+      double row[10];
+      if (tab && n < kCoshLds) {
+#pragma unroll
+        for (int i = 0; i < 10; ++i) row[i] = tab[10 * n + i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 10; ++i) row[i] = kCoshTable.v[10 * n + i];
+      }
+      series::for_lambda([&](auto i) {
+        constexpr int I = decltype(i)::value;
+        constexpr double zmax = lambda2(I) * .0625;
+        const double z = lambda2(I) * R2;
+        const double ch = series::sum<series::degree(zmax, 2), 2, 0>(z);
+        const double sh = series::sum<series::degree(zmax, 2, 1), 2, 1>(z);
+        s[I] = w[I] * __builtin_fma(row[2 * I], ch, (row[2 * I + 1] * r) * sh);
+      });
+    } else {
+      const double t = v * v;
+#pragma unroll 1
+      for (int i = 0; i < 5; ++i) {
+        const double l = i == 0 ? kLambda[0] : i == 1 ? kLambda[1] : i == 2 ? kLambda[2] : i == 3 ? kLambda[3] : kLambda[4];
+        const double vm = __builtin_fma(-l, h, v), vp = __builtin_fma(l, h, v);
+        const double e = math::exp_bounded(__builtin_fma(-vm, vm, t)) +
+                         math::exp_bounded(__builtin_fma(-vp, vp, t));
+#pragma unroll
+        for (int k = 0; k < 5; ++k) s[k] = k == i ? e : s[k];
+      }
+    }
+  }
+  __device__ double value(double p) const { return p; }
 };
 
 // exp(-sum a_i |x_i - u_i|)
@@ -298,35 +576,46 @@ struct C0 {
   {
     return static_cast<double>(math::exp_neg(static_cast<Real>(-s)));
   }
-  // The points v -+ delta of one axis change |v| by -+delta when they stay
-  // on v's side of the kink: factors e^delta (toward 0) and e^-delta (away),
-  // one exponential and its reciprocal.  A point across the kink (delta >
-  // |v|) has e^(2|v| - delta) = (e^-delta e^|v|) e^|v|, with aux = e^|v|
-  // (|v| <= 650 where the factored form is taken, so aux stays finite and
-  // the first product is at most 1).
-  // (FP64 integrands only: for an FP32 one the extra registers cost more
-  // than the exponentials they save)
-  template <class R = Real, std::enable_if_t<std::is_same_v<R, double>, int> = 0>
-  __device__ double axis_aux(int, double v) const
+  // The points v -+ l h of one axis change |v| by -+l|h| while they stay on
+  // v's side of the kink: factors e^(l|h|) and e^(-l|h|), functions of the
+  // width alone, so a region forms an exponential only for the axes that
+  // reach the kink.  There (l|h| > |v|) the near point has e^(2|v| - l|h|) =
+  // (e^(-l|h|) e^|v|) e^|v| (|v| <= 650 where the factored form is taken, so
+  // e^|v| stays finite and the first product is at most 1).
+  struct Centre {
+    double sum = 0.0;
+    __device__ void add(const C0&, int, double c, double) { sum += __builtin_fabs(c); }
+    __device__ bool safe(const C0& f) const { return f.factor_safe(sum); }
+    __device__ double value(const C0&) const { return math::exp_bounded(-sum); }
+  };
+  static constexpr int kWidthValues = 10, kTableSize = 0;
+  __device__ double width_arg(int, double h) const { return h; }
+  __device__ void width_values(double h, double (&w)[10]) const
   {
-    return math::exp_factor(__builtin_fabs(v), Real());
-  }
-  template <class R = Real, std::enable_if_t<std::is_same_v<R, double>, int> = 0>
-  __device__ void factor_pair(int, double v, double delta, double aux, double& fm,
-                              double& fp) const
-  {
-    const double e = math::exp_factor(-delta, Real());
-    const double r = math::recip(e);
-    const double across = (e * aux) * aux;
-    const bool cross = delta > __builtin_fabs(v);
-    if (v >= 0.0) {
-      fm = cross ? across : r;
-      fp = e;
-    } else {
-      fm = e;
-      fp = cross ? across : r;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      w[2 * i] = math::exp_bounded(-(kLambda[i] * __builtin_fabs(h)));
+      w[2 * i + 1] = math::recip(w[2 * i]);
     }
   }
+  template <class R = Real, if_double<R> = 0>
+  __device__ void pair_sums(int, double v, double h, const double* w, const double*,
+                            double (&s)[5]) const
+  {
+#pragma clang fp contract(off)
+    const double av = __builtin_fabs(v), ah = __builtin_fabs(h);
+#pragma unroll
+    for (int i = 0; i < 5; ++i) s[i] = w[2 * i] + w[2 * i + 1];
+    if (kLambda[0] * ah > av) {  // lambda1 is the largest
+      const double aux = math::exp_bounded(av);
+#pragma unroll
+      for (int i = 0; i < 5; ++i) {
+        const double across = w[2 * i] + (w[2 * i] * aux) * aux;
+        s[i] = kLambda[i] * ah > av ? across : s[i];
+      }
+    }
+  }
+  __device__ double value(double p) const { return p; }
   // outer(s + d) = outer(s) e^-d, non-negative terms (see Gaussian)
   static constexpr bool exponential = true;
   __device__ double factor(double d) const { return math::exp_factor(-d, Real()); }
@@ -369,7 +658,7 @@ struct Discontinuous {
 #pragma unroll
     for (int i = 1; i < D; ++i) {
       m = math::fmax_(m, t[i]);
-      s += a[i] * t[i];
+      s = math::fma_(a[i], t[i], s);
     }
     const Real v = math::exp_bounded(static_cast<Real>(c) + s);
     return m > Real(0) ? Real(0) : v;
@@ -397,6 +686,40 @@ struct Discontinuous {
     fm = factor(-static_cast<double>(a[j]) * delta);
     fp = math::recip(fm);
   }
+  // the same two factors, functions of the width alone, summed over the valid
+  // points
+  struct Centre {
+    double sum = 0.0;
+    __device__ void add(const Discontinuous& f, int j, double t, double)
+    {
+      sum = __builtin_fma(static_cast<double>(f.a[j]), t, sum);
+    }
+    __device__ bool safe(const Discontinuous& f) const { return f.factor_safe(sum); }
+    __device__ double value(const Discontinuous& f) const { return math::exp_bounded(f.c + sum); }
+  };
+  static constexpr int kWidthValues = 10, kTableSize = 0;
+  __device__ double width_arg(int j, double h) const { return static_cast<double>(a[j]) * h; }
+  __device__ void width_values(double ah, double (&w)[10]) const
+  {
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      w[2 * i] = math::exp_bounded(-(kLambda[i] * ah));
+      w[2 * i + 1] = math::recip(w[2 * i]);
+    }
+  }
+  template <class R = Real, if_double<R> = 0>
+  __device__ void pair_sums(int j, double t, double h, const double* w, const double*,
+                            double (&s)[5]) const
+  {
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+      const bool m = valid(j, __builtin_fma(-kLambda[i], h, t));
+      const bool p = valid(j, __builtin_fma(kLambda[i], h, t));
+      s[i] = (m ? w[2 * i] : 0.0) + (p ? w[2 * i + 1] : 0.0);
+    }
+  }
+  __device__ double value(double p) const { return p; }
   __device__ bool factor_safe(double s0) const
   {
     return __builtin_fabs(c + s0) <= kFactorRange<Real> - (sizeof(Real) == 8 ? 100.0 : 20.0);

@@ -1,0 +1,73 @@
+"""The pair sums (pair_region) and the corner peak's group sums (group_sums)
+against the oracle at the kernel's own points, where they can go wrong: widths
+in and out of the width tables (powers of two from 1 down past the last
+table entry, and widths that are no power of two), the Gaussian's cosh table
+at its ends and past it, lists that end inside a tile and a workgroup, and
+regions out of the sums' range among regions within it.
+
+Tolerances are test_gpu_eval's: 1e-13 of each region's scale plus the FP64
+floor of f at those points, and the error and split-axis rules given there.
+"""
+import numpy as np
+import pytest
+
+import oracle_api as O
+from test_gpu_eval import check_region_parity, genz_params, gpu_eval
+
+pytestmark = pytest.mark.gpu
+
+
+def _compare(pg, gpu, family, a, u, L, H, slices=1):
+    d, n = L.shape
+    L, H = np.ascontiguousarray(L.ravel()), np.ascontiguousarray(H.ravel())
+    with pg.Workspace(d, 0) as ws:
+        ws.set_slices(slices)
+        ge, gerr, gdim = gpu_eval(ws, gpu, family, a, u, L, H, n)
+    oe, oerr, odim, fd, rs = O.eval_regions_kform(d, family, O.params(a, u), L, H, n)
+    check_region_parity(d, family, ge, gerr, gdim, oe, oerr, odim, fd, rs, floor=True)
+
+
+def _boxes(rng, H):
+    return np.floor(rng.random(H.shape) / H) * H
+
+
+@pytest.mark.parametrize("family", ["gaussian", "c0", "discontinuous", "product_peak"])
+@pytest.mark.parametrize("d,n", [(2, 1), (2, 64 * 8 + 1), (3, 255), (5, 321), (8, 700), (10, 130)])
+@pytest.mark.parametrize("third", [False, True])
+def test_widths_in_and_out_of_the_tables(pg, gpu, family, d, n, third):
+    rng = np.random.default_rng(1000 * d + n)
+    a, u = genz_params(family, d, seed=17 + d)
+    H = 0.5 ** rng.integers(0, 14 if d < 5 else 16, size=(d, n))
+    if third:
+        H = np.where(rng.random((d, n)) < 0.5, H / 3, H)
+    _compare(pg, gpu, family, a, u, _boxes(rng, H), H)
+
+
+@pytest.mark.parametrize("d", [2, 8])
+def test_gaussian_at_the_ends_of_its_table(pg, gpu, d):
+    # y = 2 a^2 (c - u) h from 0 past the table's 100, the centre's sum
+    # within the factored range on most regions
+    n = 640
+    rng = np.random.default_rng(d)
+    a, u = [25.0] + [4.0] * (d - 1), [0.5] * d
+    H = np.full((d, n), 0.125)
+    H[0] = np.linspace(0.01, 0.9, n)
+    L = rng.random((d, n)) * (1.0 - H)
+    y = 2 * a[0] ** 2 * np.abs(L[0] + H[0] / 2 - u[0]) * H[0]
+    assert (y > 100).any() and (y < 100).any() and ((y > 99) & (y < 101)).any()
+    _compare(pg, gpu, "gaussian", a, u, L, H)
+
+
+@pytest.mark.parametrize("d", [2, 3, 5, 8])
+@pytest.mark.parametrize("slices", [1, 2, 4, 8])
+@pytest.mark.parametrize("first", [9.0, 1e31])
+def test_corner_peak_groups(pg, gpu, d, slices, first):
+    # a base past 1e30 leaves the groups' range: with the large coefficient
+    # only the boxes at the origin stay within it, in one wave with the others
+    n = 64 * 3 + 5
+    rng = np.random.default_rng(10 * d + slices)
+    a = [first] + [0.05] * (d - 1)
+    H = 0.5 ** rng.integers(1, 7, size=(d, n))
+    L = _boxes(rng, H)
+    L[0, ::3] = 0.0
+    _compare(pg, gpu, "corner_peak", a, [0.0] * d, L, H, slices)
