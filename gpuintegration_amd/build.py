@@ -41,10 +41,11 @@ HIP_SOURCES = {
     "mcubes.hip": [],
     "noalloc.hip": [],
     "segments.hip": [],
+    "small_loop.hip": [],
 }
 # sources compiled in several parts (one object each, -DPAGANI_PART=k), side
 # by side: their kernel instantiations take minutes in one
-PARTS = {"genz_eval.hip": 6, "segments.hip": 3}
+PARTS = {"genz_eval.hip": 6, "segments.hip": 3, "small_loop.hip": 4}
 CXX_SOURCES = {"rule.cpp": ["-O2", "-ffp-contract=off"],
                "mcubes_grid.cpp": ["-O2", "-ffp-contract=off"]}
 

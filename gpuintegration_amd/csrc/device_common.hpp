@@ -1,6 +1,7 @@
-// device_common.hpp -- deterministic reductions and the per-region
-// refinement, shared by the phase kernels (phases.hip) and the batch's
-// segment kernel (segments.hip).  Compile with -ffp-contract=off: the
+// device_common.hpp -- deterministic reductions, the per-region refinement
+// and the move of a kept region, shared by the phase kernels (phases.hip),
+// the batch's segment kernel (segments.hip) and the small-list loop
+// (small_loop.hip).  Compile with -ffp-contract=off: the
 // refinement is plain IEEE double in the reference's operation order.
 #pragma once
 
@@ -92,6 +93,70 @@ __device__ __forceinline__ void refine_region(double e, double r, double es, dou
   const bool pass = relerr && r < fmax(epsrel * fabs(e), 1e-200);
   r_out = r;
   active = !pass;
+}
+
+// Row `row` of a list's bounds along axis j at stride `stride`: lower bound
+// and width (from the level when lv.on), and the width's level.
+__device__ __forceinline__ void read_row(const double* __restrict__ L,
+                                         const double* __restrict__ H, const Levels& lv,
+                                         std::size_t o, int j, double& l, double& w, int& lev)
+{
+  l = L[o];
+  if (lv.on) {
+    lev = reinterpret_cast<const std::uint16_t*>(H)[o];
+    w = __builtin_ldexp(lv.h0[j], -lev);
+  } else {
+    lev = 0;
+    w = H[o];
+  }
+}
+
+// The kept region t of an n-region list (split form when pdim is given)
+// becomes parent i of the next list's m: its own bounds, derived from its
+// parent's as the evaluation derives them, at [j*m + i], the axis it is to
+// be halved along (dim[t]) and its estimate.
+template <int D>
+__device__ __forceinline__ void move_region(
+    std::size_t n, std::size_t m, std::size_t t, std::size_t i, const double* __restrict__ L,
+    const double* __restrict__ H, const std::uint8_t* __restrict__ pdim,
+    const double* __restrict__ est, const std::uint8_t* __restrict__ dim, double* __restrict__ L2,
+    double* __restrict__ H2, std::uint8_t* __restrict__ pdim2, double* __restrict__ pest,
+    const Levels& lv)
+{
+  const double ev = est[t];
+  const std::uint8_t b = dim[t];
+  // the row this region's bounds come from, and the axis its parent halves
+  // (none for a flat list)
+  const std::size_t h = n / 2;
+  std::size_t row = t, stride = n;
+  int axis = -1;
+  bool right = false;
+  if (pdim) {
+    right = t >= h;
+    row = right ? t - h : t;
+    stride = h;
+    axis = pdim[row];
+  }
+#pragma unroll
+  for (int j = 0; j < D; ++j) {
+    double l, w;
+    int g;
+    read_row(L, H, lv, static_cast<std::size_t>(j) * stride + row, j, l, w, g);
+    if (j == axis) {
+      const double half = w / 2;
+      if (right) l = l + half;
+      w = half;
+      ++g;
+    }
+    const std::size_t o = static_cast<std::size_t>(j) * m + i;
+    L2[o] = l;
+    if (lv.on)
+      reinterpret_cast<std::uint16_t*>(H2)[o] = static_cast<std::uint16_t>(g);
+    else
+      H2[o] = w;
+  }
+  pdim2[i] = b;
+  pest[i] = ev;
 }
 
 }  // namespace phases

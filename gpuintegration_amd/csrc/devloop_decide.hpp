@@ -7,9 +7,10 @@
 // holds.  While the region list is small and the memory model far from its
 // budget, those decisions need nothing but the iteration's sums, so they run
 // on the device, in one thread of the workgroup that finishes the
-// iteration's reductions last (k_step_dev), before the filter + split of the
-// same iteration; the host queues whole rounds of iterations and reads the
-// state back once per round.  Everything the device cannot decide alone --
+// iteration's reductions last (k_step_dev) or in the one workgroup that runs
+// the whole loop on short lists (k_small_loop), before the filter + split of
+// the same iteration; the host queues whole rounds of iterations and reads
+// the state back once per round.  Everything the device cannot decide alone --
 // the error-budget fix (Workspace.cuh:121-146), a memory model past a tenth
 // of its budget (where the heuristic classifier may run, :74-118), a next
 // list beyond the device loop's capacity -- stops the loop with kDevHost
@@ -110,7 +111,8 @@ __device__ __forceinline__ void decide_step(DevLoop* s, double iter_est, double 
     // grids for round_cap regions: an iteration that needs another slice
     // count (idle waves would take the place of working ones) or a larger
     // grid waits for the next round
-    if (static_cast<std::int32_t>(s->it.slices) != s->launch_slices || 2 * m > s->round_cap)
+    if ((!s->any_slices && static_cast<std::int32_t>(s->it.slices) != s->launch_slices) ||
+        2 * m > s->round_cap)
       s->it.run = 0;
   }
   if (!s->user_regions) s->cum_iters++;

@@ -25,6 +25,7 @@
 #include "phases.hpp"
 #include "classify_search.hpp"
 #include "rule.hpp"
+#include "small_loop.hpp"
 
 #include "ws_internal.hpp"
 
@@ -347,6 +348,18 @@ struct RoundGraphs {
   }
 };
 
+// The integrand of a Genz descriptor as an evaluation callback.
+struct GenzCtx {
+  pagani_genz g;
+  int precision;
+};
+
+int genz_trampoline(void* ctx, const pagani_eval_args* a)
+{
+  const GenzCtx* c = static_cast<const GenzCtx*>(ctx);
+  return pagani_genz_eval_launch(&c->g, c->precision, a);
+}
+
 // What a device-resident segment ended with (see run_device_segment).
 enum DevOutcome { kSegHost, kSegDone, kSegEmpty, kSegLimit };
 
@@ -359,9 +372,11 @@ struct LoopVars {
   Classifier* clf;
 };
 
-// Run iterations on the device, in rounds of 2, 4, 8, 16 queued
-// iterations with one host round trip each, until the device loop stops.
-// Each iteration is three launches: the evaluation, k_step_dev (refinement,
+// Run iterations on the device, with one host round trip per round, until
+// the device loop stops.  A round over a short list of an FP64 Genz integrand
+// (small_cap) is one launch of k_small_loop; other rounds queue 2, 4, 8, 16
+// iterations.
+// A queued iteration is three launches: the evaluation, k_step_dev (refinement,
 // the reductions and the decisions) and the filter + split, with fixed
 // launch shapes for the round, reading the counts from the DevLoop
 // descriptors.  On return the loop variables
@@ -439,68 +454,107 @@ int run_device_segment(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double eps
   args.dev = &ws->d_loop->it;
   make_consts(ws, lows, highs, cap, args.consts, &ws->lv);
   RoundGraphs graphs;
-
-  for (int queued = 2;; queued = std::min(queued * 2, kDevQueueMax)) {
-    // A round's launches have as many waves per workgroup as its first
-    // iteration's slice count, and grids for the largest list with that
-    // slice count (workgroups past the actual list return at once; queued
-    // iterations after the loop stops return at once too, so the grids are
-    // kept no larger than they can be used).  decide_step pauses the round
-    // (it.run = 0, status kDevRun) before an iteration with another slice
-    // count.
-    h.it.run = 1;
-    h.launch_slices = static_cast<std::int32_t>(h.it.slices);
-    h.round_cap = round_cap(ws, h.it.n, cap, h.launch_slices);
-    set_slices(args.consts, h.launch_slices);
-    args.n = h.round_cap;
-    const std::size_t rcap = h.round_cap;
-    HIP_TRY(ws, hipMemcpyAsync(ws->d_loop, ws->h_loop, sizeof(DevLoop), hipMemcpyHostToDevice,
-                               ws->stream));
-    if (ws->timing) record(ws, EV_DEV0);
-    // the round's launches: `queued` iterations of evaluation, refinement
-    // with reductions and decisions, filter + split
-    auto enqueue = [&]() -> int {
-      for (int q = 0; q < queued; ++q) {
-        const int erc = eval(ctx, &args);
-        if (erc) return fail(ws, erc < 0 ? erc : PAGANI_EHIP, "evaluation callback failed");
-        HIP_TRY(ws, ph::step_dev(ws->stream, rcap, ws->d_loop, ws->est.p, ws->err0.p,
-                                 ws->err1.p, ws->pest.p, epsrel, relerr, ws->active.p, ws->part.p,
-                                 ws->cnt.p, ws->off.p, ws->fpart.p, ws->fcnt.p, ws->foff.p,
-                                 ws->d_scal, &ws->d_loop->ticket));
-        HIP_TRY(ws, ph::compact_dev(ws->stream, rcap, &ws->d_loop->cp, d, ws->L[0].p,
-                                    ws->H[0].p, ws->L[1].p, ws->H[1].p, ws->pdim[0].p,
-                                    ws->pdim[1].p, ws->active.p, ws->est.p, ws->err0.p,
-                                    ws->err1.p, ws->dim.p, ws->off.p, ws->foff.p, ws->pest.p,
-                                    nullptr, ws->lv));
+  const GenzCtx* genz = eval == genz_trampoline ? static_cast<const GenzCtx*>(ctx) : nullptr;
+  const std::uint64_t scap =
+      genz && genz->precision == PAGANI_FP64 ? small_cap(genz->g.family, d) : 0;
+  const SmallBufs sb{{ws->L[0].p, ws->L[1].p},
+                     {ws->H[0].p, ws->H[1].p},
+                     {ws->pdim[0].p, ws->pdim[1].p},
+                     ws->est.p,
+                     ws->err0.p,
+                     ws->err1.p,
+                     ws->pest.p,
+                     ws->dim.p,
+                     ws->active.p,
+                     ws->off.p,
+                     ws->foff.p,
+                     ws->d_scal,
+                     ws->lv};
+  // the launches of a round, eagerly or -- `captured` -- as a graph kept
+  // under (rcap, slices)
+  auto launch = [&](bool captured, std::uint64_t rcap, int slices, auto&& enqueue) -> int {
+    if (!captured) return enqueue();
+    hipGraphExec_t exec = graphs.find(rcap, slices);
+    if (!exec) {
+      HIP_TRY(ws, hipStreamBeginCapture(ws->stream, hipStreamCaptureModeThreadLocal));
+      const int erc = enqueue();
+      hipGraph_t g = nullptr;
+      const hipError_t e = hipStreamEndCapture(ws->stream, &g);
+      if (erc) {
+        if (g) (void)hipGraphDestroy(g);
+        return erc;
       }
-      return PAGANI_OK;
-    };
-    if (ws->graphs && queued == kDevQueueMax) {
-      hipGraphExec_t exec = graphs.find(rcap, h.launch_slices);
-      if (!exec) {
-        HIP_TRY(ws, hipStreamBeginCapture(ws->stream, hipStreamCaptureModeThreadLocal));
-        rc = enqueue();
-        hipGraph_t g = nullptr;
-        const hipError_t e = hipStreamEndCapture(ws->stream, &g);
-        if (rc) {
-          if (g) (void)hipGraphDestroy(g);
-          return rc;
-        }
-        if (e != hipSuccess) return hip_fail(ws, e, "hipStreamEndCapture");
-        const hipError_t ie = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (ie != hipSuccess) return hip_fail(ws, ie, "hipGraphInstantiate");
-        graphs.entries.push_back({rcap, h.launch_slices, exec});
-      }
-      HIP_TRY(ws, hipGraphLaunch(exec, ws->stream));
-      ws->stats.graph_launches++;
-    } else if ((rc = enqueue())) {
-      return rc;
+      if (e != hipSuccess) return hip_fail(ws, e, "hipStreamEndCapture");
+      const hipError_t ie = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
+      (void)hipGraphDestroy(g);
+      if (ie != hipSuccess) return hip_fail(ws, ie, "hipGraphInstantiate");
+      graphs.entries.push_back({rcap, slices, exec});
     }
-    if (ws->timing) record(ws, EV_DEV1);
-    HIP_TRY(ws, hipMemcpyAsync(ws->h_loop, ws->d_loop, sizeof(DevLoop), hipMemcpyDeviceToHost,
-                               ws->stream));
-    HIP_TRY(ws, hipStreamSynchronize(ws->stream));
+    HIP_TRY(ws, hipGraphLaunch(exec, ws->stream));
+    ws->stats.graph_launches++;
+    return PAGANI_OK;
+  };
+
+  int queued = 2, smalls = 0;
+  for (;;) {
+    h.it.run = 1;
+    if (h.it.n <= scap) {
+      // the loop's state is read from and written back to h_loop itself
+      const int iterations = smalls ? kSmallNext : kSmallFirst;
+      h.any_slices = 1;
+      h.round_cap = scap;
+      if (ws->timing) record(ws, EV_DEV0);
+      rc = launch(ws->graphs && smalls, scap, 0, [&]() -> int {
+        HIP_TRY(ws, launch_small_loop(ws->stream, genz->g, ws->h_loop, iterations, sb,
+                                      args.consts));
+        return PAGANI_OK;
+      });
+      if (rc) return rc;
+      ++smalls;
+      if (ws->timing) record(ws, EV_DEV1);
+      HIP_TRY(ws, hipStreamSynchronize(ws->stream));
+    } else {
+      // A round's launches have as many waves per workgroup as its first
+      // iteration's slice count, and grids for the largest list with that
+      // slice count (workgroups past the actual list return at once; queued
+      // iterations after the loop stops return at once too, so the grids are
+      // kept no larger than they can be used).  decide_step pauses the round
+      // (it.run = 0, status kDevRun) before an iteration with another slice
+      // count.
+      h.any_slices = 0;
+      h.launch_slices = static_cast<std::int32_t>(h.it.slices);
+      h.round_cap = round_cap(ws, h.it.n, cap, h.launch_slices);
+      set_slices(args.consts, h.launch_slices);
+      args.n = h.round_cap;
+      const std::size_t rcap = h.round_cap;
+      HIP_TRY(ws, hipMemcpyAsync(ws->d_loop, ws->h_loop, sizeof(DevLoop), hipMemcpyHostToDevice,
+                                 ws->stream));
+      if (ws->timing) record(ws, EV_DEV0);
+      // the round's launches: `queued` iterations of evaluation, refinement
+      // with reductions and decisions, filter + split
+      rc = launch(ws->graphs && queued == kDevQueueMax, rcap, h.launch_slices, [&]() -> int {
+        for (int q = 0; q < queued; ++q) {
+          const int erc = eval(ctx, &args);
+          if (erc) return fail(ws, erc < 0 ? erc : PAGANI_EHIP, "evaluation callback failed");
+          HIP_TRY(ws, ph::step_dev(ws->stream, rcap, ws->d_loop, ws->est.p, ws->err0.p,
+                                   ws->err1.p, ws->pest.p, epsrel, relerr, ws->active.p,
+                                   ws->part.p, ws->cnt.p, ws->off.p, ws->fpart.p, ws->fcnt.p,
+                                   ws->foff.p, ws->d_scal, &ws->d_loop->ticket));
+          HIP_TRY(ws, ph::compact_dev(ws->stream, rcap, &ws->d_loop->cp, d, ws->L[0].p,
+                                      ws->H[0].p, ws->L[1].p, ws->H[1].p, ws->pdim[0].p,
+                                      ws->pdim[1].p, ws->active.p, ws->est.p, ws->err0.p,
+                                      ws->err1.p, ws->dim.p, ws->off.p, ws->foff.p, ws->pest.p,
+                                      nullptr, ws->lv));
+        }
+        return PAGANI_OK;
+      });
+      if (rc) return rc;
+      queued = std::min(queued * 2, kDevQueueMax);
+      if (ws->timing) record(ws, EV_DEV1);
+      HIP_TRY(ws, hipMemcpyAsync(ws->h_loop, ws->d_loop, sizeof(DevLoop), hipMemcpyDeviceToHost,
+                                 ws->stream));
+      HIP_TRY(ws, hipStreamSynchronize(ws->stream));
+    }
     if (ws->timing) ws->stats.device_ms += elapsed(ws, EV_DEV0, EV_DEV1);
     ws->stats.device_rounds++;
     ws->stats.device_iterations += h.iterations;
@@ -936,17 +990,6 @@ done:
       std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - wall0).count();
   *out = cum;
   return status_code;
-}
-
-struct GenzCtx {
-  pagani_genz g;
-  int precision;
-};
-
-int genz_trampoline(void* ctx, const pagani_eval_args* a)
-{
-  const GenzCtx* c = static_cast<const GenzCtx*>(ctx);
-  return pagani_genz_eval_launch(&c->g, c->precision, a);
 }
 
 int check_genz(pagani_ws* ws, const pagani_genz* f, int precision)

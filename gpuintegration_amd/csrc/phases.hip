@@ -74,22 +74,6 @@ __global__ void __launch_bounds__(256) k_to_levels(int d, std::size_t n,
   }
 }
 
-// Row `row` of a list's bounds along axis j at stride `stride`: lower bound
-// and width (from the level when lv.on), and the width's level.
-__device__ __forceinline__ void read_row(const double* __restrict__ L,
-                                         const double* __restrict__ H, const Levels& lv,
-                                         std::size_t o, int j, double& l, double& w, int& lev)
-{
-  l = L[o];
-  if (lv.on) {
-    lev = reinterpret_cast<const std::uint16_t*>(H)[o];
-    w = __builtin_ldexp(lv.h0[j], -lev);
-  } else {
-    lev = 0;
-    w = H[o];
-  }
-}
-
 // RefineError (Phases.cuh:219-268) and the relerr flag; children t and t+n/2
 // share parent t mod n/2.
 __device__ __forceinline__ void refine_chunk(std::size_t n, const double* __restrict__ est,
@@ -958,7 +942,6 @@ __device__ __forceinline__ void compact_parents_chunk(
   __shared__ std::uint16_t src[kChunk];
   std::size_t base, end;
   chunk_range(chunk, n, paired, base, end);
-  const std::size_t h = n / 2;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   bool a[kSteps];
   std::uint32_t pre[kSteps];
@@ -994,42 +977,8 @@ __device__ __forceinline__ void compact_parents_chunk(
   for (std::uint32_t q = threadIdx.x; q < kept; q += kCompactThreads) {
     const std::size_t i = first + q;
     if (i >= m) break;
-    const std::size_t t = base + src[q];
-    const double ev = est[t];
-    const double rv = perr ? err[t] : 0.0;
-    const int b = dim[t];
-    // the row this region's bounds come from, and the axis its parent
-    // halves (none for a flat list)
-    std::size_t row = t, stride = n;
-    int axis = -1;
-    bool right = false;
-    if (pdim) {
-      right = t >= h;
-      row = right ? t - h : t;
-      stride = h;
-      axis = pdim[row];
-    }
-#pragma unroll
-    for (int j = 0; j < D; ++j) {
-      double l, w;
-      int g;
-      read_row(L, H, lv, static_cast<std::size_t>(j) * stride + row, j, l, w, g);
-      if (j == axis) {
-        const double half = w / 2;
-        if (right) l = l + half;
-        w = half;
-        ++g;
-      }
-      const std::size_t o = static_cast<std::size_t>(j) * m + i;
-      L2[o] = l;
-      if (lv.on)
-        reinterpret_cast<std::uint16_t*>(H2)[o] = static_cast<std::uint16_t>(g);
-      else
-        H2[o] = w;
-    }
-    pdim2[i] = static_cast<std::uint8_t>(b);
-    pest[i] = ev;
-    if (perr) perr[i] = rv;
+    move_region<D>(n, m, base + src[q], i, L, H, pdim, est, dim, L2, H2, pdim2, pest, lv);
+    if (perr) perr[i] = err[base + src[q]];
   }
 }
 

@@ -71,9 +71,10 @@ struct DevLoop {
   std::uint64_t iters_collected;
   // the evaluation's slice choice (choose_slices, with the integrand's
   // tuned table when has_table) and this round's launch: its waves per
-  // workgroup and the largest list its grids cover
+  // workgroup (any_slices: it takes every slice count) and the largest list
+  // it covers
   std::int32_t num_cus, slices_override, generic, launch_slices;
-  std::int32_t has_table, pad_table;
+  std::int32_t has_table, any_slices;
   std::uint8_t slice_table[kSliceBuckets];
   std::uint64_t round_cap;
   // per round

@@ -803,6 +803,7 @@ __device__ __forceinline__ bool cosine_sums(F& f, const double (&cR)[D], const d
                                             double jac, const pagani_eval_consts& C,
                                             double (&rs)[PAGANI_NRULES], int& bisect)
 {
+#pragma clang fp contract(off)
   double phi0 = f.phase_angle();
   double hmax = 0.0;
 #pragma unroll
@@ -833,7 +834,8 @@ __device__ __forceinline__ bool cosine_sums(F& f, const double (&cR)[D], const d
     s1 += fa + fb;
     s2 += fc + fd;
     const double diff =
-        __builtin_fabs(base + C.ratio * (fa * jac + fb * jac) - (fc * jac + fd * jac));
+        __builtin_fabs(__builtin_fma(C.ratio, __builtin_fma(fa, jac, fb * jac), base) -
+                       __builtin_fma(fc, jac, fd * jac));
     if (diff > maxdiff) {
       maxdiff = diff;
       bisect = j;
@@ -852,7 +854,8 @@ __device__ __forceinline__ bool cosine_sums(F& f, const double (&cR)[D], const d
                                   c0 * e2, c0 * g11, c0 * e3, c0 * p5};
 #pragma unroll
   for (int r = 0; r < PAGANI_NRULES; ++r) {
-    double acc = C.w[0][r] * v[0] + C.w[1][r] * v[1] + C.w[2][r] * v[2];
+    double acc =
+        __builtin_fma(C.w[2][r], v[2], __builtin_fma(C.w[0][r], v[0], C.w[1][r] * v[1]));
 #pragma unroll
     for (int s = 3; s < PAGANI_NSETS; ++s) acc = __builtin_fma(C.w[s][r], v[s], acc);
     rs[r] = acc;
