@@ -47,6 +47,40 @@ __device__ __forceinline__ DD wave_reduce(DD v)
   return v;
 }
 
+// Four sums over a wave at once: the steps of wave_reduce, interleaved.
+__device__ __forceinline__ void wave_reduce4(DD (&v)[4])
+{
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    DD o[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o[i].hi = __shfl_xor(v[i].hi, off, 64);
+      o[i].lo = __shfl_xor(v[i].lo, off, 64);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = dd_add(v[i], o[i]);
+  }
+}
+
+// Four DDs over a 256-thread block: block_reduce's steps, interleaved, with
+// one barrier (sh is the caller's, used once).
+__device__ __forceinline__ void block_reduce4(DD (&v)[4], DD (&sh)[4][kThreads / 64])
+{
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  wave_reduce4(v);
+  if (lane == 0)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sh[i][wave] = v[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[i] = sh[i][0];
+#pragma unroll
+    for (int w = 1; w < kThreads / 64; ++w) v[i] = dd_add(v[i], sh[i][w]);
+  }
+}
+
 // Reduce a DD over a 256-thread block; every thread gets the result.
 __device__ __forceinline__ DD block_reduce(DD v, DD* sh)
 {

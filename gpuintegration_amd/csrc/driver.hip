@@ -320,31 +320,30 @@ std::uint64_t round_cap(const pagani_ws* ws, std::uint64_t n, std::uint64_t cap,
   return lo;
 }
 
-// Iterations queued per round at most: a round that stops early leaves the
-// rest as no-op launches, so the length trades round trips for those.
-constexpr int kDevQueueMax = 16;
-
 // Full-length rounds of the device-resident loop captured as HIP graphs:
 // every launch of a round is fixed by the round's length, its grids (the
 // largest list of its slice count) and its slice count, so a later round
 // with the same three replays the graph (one launch instead of 48).  Kept
-// for one segment (the buffers it points at are fixed for the segment).
+// for one segment (the buffers it points at are fixed for the segment), and
+// captured when a round comes up again: a capture takes longer than the
+// launches it replaces.
 struct RoundGraphs {
   struct Entry {
     std::uint64_t rcap;
     int slices;
-    hipGraphExec_t exec;
+    hipGraphExec_t exec;  // NULL: launched once, eagerly
   };
   std::vector<Entry> entries;
-  hipGraphExec_t find(std::uint64_t rcap, int slices) const
+  Entry* find(std::uint64_t rcap, int slices)
   {
-    for (const Entry& e : entries)
-      if (e.rcap == rcap && e.slices == slices) return e.exec;
+    for (Entry& e : entries)
+      if (e.rcap == rcap && e.slices == slices) return &e;
     return nullptr;
   }
   ~RoundGraphs()
   {
-    for (Entry& e : entries) (void)hipGraphExecDestroy(e.exec);
+    for (Entry& e : entries)
+      if (e.exec) (void)hipGraphExecDestroy(e.exec);
   }
 };
 
@@ -359,6 +358,9 @@ int genz_trampoline(void* ctx, const pagani_eval_args* a)
   const GenzCtx* c = static_cast<const GenzCtx*>(ctx);
   return pagani_genz_eval_launch(&c->g, c->precision, a);
 }
+
+// Doublings of its first list that a round's grids cover at most.
+constexpr int kRoundGrowth = 3;
 
 // What a device-resident segment ended with (see run_device_segment).
 enum DevOutcome { kSegHost, kSegDone, kSegEmpty, kSegLimit };
@@ -451,7 +453,6 @@ int run_device_segment(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double eps
   args.err = ws->err0.p;
   args.dim = ws->dim.p;
   args.stream = ws->stream;
-  args.dev = &ws->d_loop->it;
   make_consts(ws, lows, highs, cap, args.consts, &ws->lv);
   RoundGraphs graphs;
   const GenzCtx* genz = eval == genz_trampoline ? static_cast<const GenzCtx*>(ctx) : nullptr;
@@ -474,8 +475,12 @@ int run_device_segment(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double eps
   // under (rcap, slices)
   auto launch = [&](bool captured, std::uint64_t rcap, int slices, auto&& enqueue) -> int {
     if (!captured) return enqueue();
-    hipGraphExec_t exec = graphs.find(rcap, slices);
-    if (!exec) {
+    RoundGraphs::Entry* entry = graphs.find(rcap, slices);
+    if (!entry) {
+      graphs.entries.push_back({rcap, slices, nullptr});
+      return enqueue();
+    }
+    if (!entry->exec) {
       HIP_TRY(ws, hipStreamBeginCapture(ws->stream, hipStreamCaptureModeThreadLocal));
       const int erc = enqueue();
       hipGraph_t g = nullptr;
@@ -485,12 +490,14 @@ int run_device_segment(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double eps
         return erc;
       }
       if (e != hipSuccess) return hip_fail(ws, e, "hipStreamEndCapture");
-      const hipError_t ie = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
+      const hipError_t ie = hipGraphInstantiate(&entry->exec, g, nullptr, nullptr, 0);
       (void)hipGraphDestroy(g);
-      if (ie != hipSuccess) return hip_fail(ws, ie, "hipGraphInstantiate");
-      graphs.entries.push_back({rcap, slices, exec});
+      if (ie != hipSuccess) {
+        entry->exec = nullptr;
+        return hip_fail(ws, ie, "hipGraphInstantiate");
+      }
     }
-    HIP_TRY(ws, hipGraphLaunch(exec, ws->stream));
+    HIP_TRY(ws, hipGraphLaunch(entry->exec, ws->stream));
     ws->stats.graph_launches++;
     return PAGANI_OK;
   };
@@ -516,14 +523,17 @@ int run_device_segment(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double eps
     } else {
       // A round's launches have as many waves per workgroup as its first
       // iteration's slice count, and grids for the largest list with that
-      // slice count (workgroups past the actual list return at once; queued
-      // iterations after the loop stops return at once too, so the grids are
-      // kept no larger than they can be used).  decide_step pauses the round
-      // (it.run = 0, status kDevRun) before an iteration with another slice
-      // count.
+      // slice count that a few iterations can lead to (an iteration at most
+      // doubles the list; workgroups past the actual list return at once, a
+      // few us per thousand, as do the iterations queued after the loop
+      // stops).  decide_step pauses the round (it.run = 0, status kDevRun)
+      // before an iteration with another slice count or a larger list.
+      const int growth = std::min(queued - 1, kRoundGrowth);
       h.any_slices = 0;
       h.launch_slices = static_cast<std::int32_t>(h.it.slices);
-      h.round_cap = round_cap(ws, h.it.n, cap, h.launch_slices);
+      h.round_cap = std::min(round_cap(ws, h.it.n, cap, h.launch_slices),
+                             std::uint64_t(2) << (slice_bucket(h.it.n) + growth));
+      h.its[0] = h.it;
       set_slices(args.consts, h.launch_slices);
       args.n = h.round_cap;
       const std::size_t rcap = h.round_cap;
@@ -534,12 +544,12 @@ int run_device_segment(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double eps
       // with reductions and decisions, filter + split
       rc = launch(ws->graphs && queued == kDevQueueMax, rcap, h.launch_slices, [&]() -> int {
         for (int q = 0; q < queued; ++q) {
+          args.dev = &ws->d_loop->its[q];
           const int erc = eval(ctx, &args);
           if (erc) return fail(ws, erc < 0 ? erc : PAGANI_EHIP, "evaluation callback failed");
-          HIP_TRY(ws, ph::step_dev(ws->stream, rcap, ws->d_loop, ws->est.p, ws->err0.p,
+          HIP_TRY(ws, ph::step_dev(ws->stream, rcap, ws->d_loop, q, ws->est.p, ws->err0.p,
                                    ws->err1.p, ws->pest.p, epsrel, relerr, ws->active.p,
-                                   ws->part.p, ws->cnt.p, ws->off.p, ws->fpart.p, ws->fcnt.p,
-                                   ws->foff.p, ws->d_scal, &ws->d_loop->ticket));
+                                   ws->part.p, ws->cnt.p, ws->off.p, ws->foff.p, ws->d_scal));
           HIP_TRY(ws, ph::compact_dev(ws->stream, rcap, &ws->d_loop->cp, d, ws->L[0].p,
                                       ws->H[0].p, ws->L[1].p, ws->H[1].p, ws->pdim[0].p,
                                       ws->pdim[1].p, ws->active.p, ws->est.p, ws->err0.p,

@@ -22,23 +22,18 @@ __device__ __forceinline__ void write_record(DD s0, DD s1, DD s2, DD s3, std::ui
                                              double* part, std::uint32_t* cnt,
                                              std::size_t chunk = blockIdx.x)
 {
-  __shared__ DD sh[kThreads / 64];
+  __shared__ DD sh[4][kThreads / 64];
   __shared__ std::uint32_t shc[kThreads / 64];
-  s0 = block_reduce(s0, sh);
-  s1 = block_reduce(s1, sh);
-  s2 = block_reduce(s2, sh);
-  s3 = block_reduce(s3, sh);
+  DD v[4] = {s0, s1, s2, s3};
+  block_reduce4(v, sh);
   c = block_count(c, shc);
   if (threadIdx.x == 0) {
     double* p = part + chunk * kPartDoubles;
-    p[0] = s0.hi;
-    p[1] = s0.lo;
-    p[2] = s1.hi;
-    p[3] = s1.lo;
-    p[4] = s2.hi;
-    p[5] = s2.lo;
-    p[6] = s3.hi;
-    p[7] = s3.lo;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      p[2 * i] = v[i].hi;
+      p[2 * i + 1] = v[i].lo;
+    }
     if (cnt) cnt[chunk] = c;
   }
 }
@@ -74,22 +69,26 @@ __global__ void __launch_bounds__(256) k_to_levels(int d, std::size_t n,
   }
 }
 
-// RefineError (Phases.cuh:219-268) and the relerr flag; children t and t+n/2
-// share parent t mod n/2.
-__device__ __forceinline__ void refine_chunk(std::size_t n, const double* __restrict__ est,
-                                             const double* err_in, double* err_out,
-                                             const double* __restrict__ pest, double epsrel,
-                                             int relerr, std::uint8_t* __restrict__ active,
-                                             double* __restrict__ part,
-                                             std::uint32_t* __restrict__ cnt,
-                                             std::size_t chunk = blockIdx.x)
+// RefineError (Phases.cuh:219-268) and the relerr flag of a chunk's regions;
+// children t and t+n/2 share parent t mod n/2.  Each thread returns its
+// share of the chunk's record: the sums of estimates and errors, of all
+// regions and of the active ones, the active count and the errors' minimum
+// and maximum.
+__device__ __forceinline__ void refine_regions(std::size_t n, const double* __restrict__ est,
+                                               const double* err_in, double* err_out,
+                                               const double* __restrict__ pest, double epsrel,
+                                               int relerr, std::uint8_t* __restrict__ active,
+                                               std::size_t chunk, DD (&v)[4], std::uint32_t& c,
+                                               double& mn, double& mx)
 {
   std::size_t base, end;
   chunk_range(chunk, n, pest != nullptr, base, end);
   const std::size_t h = n / 2;
-  DD se{0, 0}, sr{0, 0}, sae{0, 0}, sar{0, 0};
-  std::uint32_t c = 0;
-  double mn = HUGE_VAL, mx = -HUGE_VAL;  // of the refined errors
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = DD{0, 0};
+  c = 0;
+  mn = HUGE_VAL;
+  mx = -HUGE_VAL;
 #pragma unroll
   for (int k = 0; k < kPerThread; ++k) {
     const std::size_t t = base + static_cast<std::size_t>(k) * kThreads + threadIdx.x;
@@ -105,18 +104,31 @@ __device__ __forceinline__ void refine_chunk(std::size_t n, const double* __rest
       }
       err_out[t] = r;
       active[t] = a ? 1 : 0;
-      se = dd_add(se, e);
-      sr = dd_add(sr, r);
+      v[0] = dd_add(v[0], e);
+      v[1] = dd_add(v[1], r);
       mn = fmin(mn, r);
       mx = fmax(mx, r);
       if (a) {
-        sae = dd_add(sae, e);
-        sar = dd_add(sar, r);
+        v[2] = dd_add(v[2], e);
+        v[3] = dd_add(v[3], r);
         ++c;
       }
     }
   }
-  write_record(se, sr, sae, sar, c, part, cnt, chunk);
+}
+
+__device__ __forceinline__ void refine_chunk(std::size_t n, const double* __restrict__ est,
+                                             const double* err_in, double* err_out,
+                                             const double* __restrict__ pest, double epsrel,
+                                             int relerr, std::uint8_t* __restrict__ active,
+                                             double* __restrict__ part,
+                                             std::uint32_t* __restrict__ cnt, std::size_t chunk)
+{
+  DD v[4];
+  std::uint32_t c;
+  double mn, mx;
+  refine_regions(n, est, err_in, err_out, pest, epsrel, relerr, active, chunk, v, c, mn, mx);
+  write_record(v[0], v[1], v[2], v[3], c, part, cnt, chunk);
   // the errors' minimum and maximum in the record's last two slots, as
   // k_minmax writes them: the classifier's search range without a pass of
   // its own when it runs on these errors
@@ -472,11 +484,9 @@ __device__ __forceinline__ void fold_block(std::size_t fold, std::size_t nchunks
                                            const std::uint32_t* __restrict__ cnt,
                                            std::uint64_t* __restrict__ off,
                                            double* __restrict__ fpart,
-                                           std::uint32_t* __restrict__ fcnt, int with_minmax,
-                                           DD* sums_out = nullptr,
-                                           std::uint32_t* total_out = nullptr)
+                                           std::uint32_t* __restrict__ fcnt, int with_minmax)
 {
-  __shared__ DD sh[kThreads / 64];
+  __shared__ DD sh[4][kThreads / 64];
   __shared__ std::uint32_t wtot[kThreads / 64];
   __shared__ double smn[kThreads / 64], smx[kThreads / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -495,8 +505,7 @@ __device__ __forceinline__ void fold_block(std::size_t fold, std::size_t nchunks
     }
     if (cnt) v = cnt[c];
   }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) s[i] = block_reduce(s[i], sh);
+  block_reduce4(s, sh);
   if (cnt) {
     std::uint32_t inc = v;
 #pragma unroll
@@ -514,7 +523,6 @@ __device__ __forceinline__ void fold_block(std::size_t fold, std::size_t nchunks
     }
     if (live && off) off[c] = wbase + inc - v;
     if (threadIdx.x == 0) fcnt[fold] = total;
-    if (total_out) *total_out = total;
   }
   if (with_minmax) {
 #pragma unroll
@@ -542,10 +550,6 @@ __device__ __forceinline__ void fold_block(std::size_t fold, std::size_t nchunks
     }
     q[8] = mn;
     q[9] = mx;
-  }
-  if (sums_out) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) sums_out[i] = s[i];
   }
 }
 
@@ -733,52 +737,112 @@ __global__ void __launch_bounds__(kFinThreads)
   finalize_block(nchunks, part, cnt, off, out, with_minmax);
 }
 
-// One step of the device-resident loop after the evaluation: the
-// refinement of every chunk (k_refine's work), then -- in whichever
-// workgroup finishes last -- the fold of the chunk records (k_fold's work
-// for the single fold a list of at most kDevLoopMax regions has), the final
-// sums exactly as k_finalize forms them from one fold record, and the
-// iteration's decisions (decide_step).  All workgroups of the grid take a
-// ticket, those past the list too, so the descriptor the decision rewrites
-// has been read by every workgroup before it changes.
-__global__ void __launch_bounds__(kThreads)
-    k_step_dev(internal::DevLoop* __restrict__ loop, const double* __restrict__ est,
-               double* err0, double* err1, const double* __restrict__ pest, double epsrel,
-               int relerr, std::uint8_t* __restrict__ active, double* __restrict__ part,
-               std::uint32_t* __restrict__ cnt, std::uint64_t* __restrict__ off,
-               double* __restrict__ fpart, std::uint32_t* __restrict__ fcnt,
-               std::uint64_t* __restrict__ foff, Scalars* __restrict__ sc,
-               std::uint32_t* __restrict__ ticket)
+// One step of the device-resident loop after the evaluation, queued as the
+// round's q-th: the refinement of every chunk (k_refine's work), then -- in
+// whichever workgroup finishes last -- the fold of the chunk records (k_fold's
+// work for the single fold a list of at most kDevLoopMax regions has), the
+// final sums as k_finalize forms them from one fold record (its further steps
+// add zero to a normalised sum) and the iteration's decisions (decide_step).
+//
+// Bound by latency: a few workgroups of 4096 regions and a chain of memory
+// round trips.  The list is described in its[q], written by the step before
+// and by nobody during this one, so workgroups past the list return without
+// a ticket.  A chunk's record goes out in agent-scope stores, which are
+// written through to where every XCD sees them; waiting for those stores and
+// nothing else replaces a release, whose write-back of the whole L2 also
+// carries the chunk's errors and flags (needed by later launches only).  The
+// loop's state is copied to LDS and back by all lanes, so that the decisions,
+// one lane's, wait for no memory.
+__device__ __forceinline__ void store_agent(double* p, double v)
 {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double load_agent(const double* p)
+{
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ void __launch_bounds__(kThreads)
+    k_step_dev(internal::DevLoop* __restrict__ loop, int q, const double* __restrict__ est,
+               double* err0, double* err1, const double* __restrict__ pest, double epsrel,
+               int relerr, std::uint8_t* __restrict__ active, double* part, std::uint32_t* cnt,
+               std::uint64_t* __restrict__ off, std::uint64_t* __restrict__ foff,
+               Scalars* __restrict__ sc)
+{
+  __shared__ internal::DevLoop sh;
+  __shared__ DD shd[2][4][kThreads / 64];
+  __shared__ std::uint32_t shc[kThreads / 64], wtot[kThreads / 64];
   __shared__ int last;
-  const pagani_dev_iter it = loop->it;
+  const pagani_dev_iter it = loop->its[q];
   if (!it.run) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) loop->cp.run = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      loop->cp.run = 0;
+      loop->its[q + 1] = it;
+    }
     return;
   }
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const std::size_t n = it.n;
   const bool parents = it.has_parents != 0;
   const std::size_t nch = num_chunks(n, parents);
-  if (blockIdx.x < nch)
-    refine_chunk(n, est, err0, parents ? err1 : err0, parents ? pest : nullptr, epsrel, relerr,
-                 active, part, cnt, paired_chunk(blockIdx.x, nch));
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0) last = atomicAdd(ticket, 1u) == gridDim.x - 1 ? 1 : 0;
+  if (blockIdx.x >= nch) return;
+  const std::size_t chunk = paired_chunk(blockIdx.x, nch);
+  DD v[4];
+  std::uint32_t c;
+  double mn, mx;
+  refine_regions(n, est, err0, parents ? err1 : err0, parents ? pest : nullptr, epsrel, relerr,
+                 active, chunk, v, c, mn, mx);
+  block_reduce4(v, shd[0]);
+  c = block_count(c, shc);
+  if (tid == 0) {
+    double* p = part + chunk * kPartDoubles;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      store_agent(p + 2 * i, v[i].hi);
+      store_agent(p + 2 * i + 1, v[i].lo);
+    }
+    __hip_atomic_store(cnt + chunk, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // the stores above have reached memory before the ticket is taken
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    last = __hip_atomic_fetch_add(&loop->ticket, 1u, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT) == nch - 1;
+    asm volatile("" ::: "memory");
+  }
   __syncthreads();
   if (!last) return;
-  __threadfence();
-  DD fs[4];
-  std::uint32_t total = 0;
-  fold_block(0, nch, part, cnt, off, fpart, fcnt, 0, fs, &total);
-  if (threadIdx.x == 0) {
+  constexpr int kHead = offsetof(internal::DevLoop, trace) / 4;
+  std::uint32_t* w = reinterpret_cast<std::uint32_t*>(loop);
+  std::uint32_t* ws = reinterpret_cast<std::uint32_t*>(&sh);
+  for (int i = tid; i < kHead; i += kThreads) ws[i] = w[i];
+  std::uint32_t k = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = DD{0, 0};
+  if (static_cast<std::size_t>(tid) < nch) {
+    const double* p = part + static_cast<std::size_t>(tid) * kPartDoubles;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = DD{load_agent(p + 2 * i), load_agent(p + 2 * i + 1)};
+    k = __hip_atomic_load(cnt + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  std::uint32_t inc = k;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const std::uint32_t y = __shfl_up(inc, o, 64);
+    if (lane >= o) inc += y;
+  }
+  if (lane == 63) wtot[wave] = inc;
+  block_reduce4(v, shd[1]);
+  std::uint32_t wbase = 0, total = 0;
+#pragma unroll
+  for (int i = 0; i < kThreads / 64; ++i) {
+    if (i < wave) wbase += wtot[i];
+    total += wtot[i];
+  }
+  if (static_cast<std::size_t>(tid) < nch) off[tid] = wbase + inc - k;
+  if (tid == 0) {
     double sums[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      // k_finalize over one fold record: its thread 0 adds the record to
-      // zero, then meets only zeros on the way up its tree
-      DD x = dd_add(DD{0.0, 0.0}, DD{fs[i].hi, fs[i].lo});
-      for (int stride = kFinThreads / 2; stride > 0; stride >>= 1) x = dd_add(x, DD{0.0, 0.0});
+      const DD x = dd_add(DD{0.0, 0.0}, v[i]);
       sums[i] = x.hi + x.lo;
       sc->sum[i] = sums[i];
     }
@@ -787,9 +851,14 @@ __global__ void __launch_bounds__(kThreads)
     sc->mn = 0.0;
     sc->mx = 0.0;
     sc->pad = 0;
-    internal::decide_step(loop, sums[0], sums[1], sums[2], sums[3], total);
-    *ticket = 0;
+    const std::uint32_t nt = sh.ntrace;
+    internal::decide_step(&sh, sums[0], sums[1], sums[2], sums[3], total);
+    if (sh.ntrace > nt) loop->trace[nt] = sh.trace[nt];
+    sh.ticket = 0;
+    loop->its[q + 1] = sh.it;
   }
+  __syncthreads();
+  for (int i = tid; i < kHead; i += kThreads) w[i] = ws[i];
 }
 
 // Chunk-local exclusive position of the active element t (ballot within the
@@ -1263,17 +1332,16 @@ hipError_t compact(hipStream_t s, int split, int d, std::size_t n, std::size_t m
   });
 }
 
-hipError_t step_dev(hipStream_t s, std::size_t n_cap, internal::DevLoop* loop, const double* est,
-                    double* err0, double* err1, const double* pest, double epsrel, int relerr,
-                    std::uint8_t* active, double* part, std::uint32_t* cnt, std::uint64_t* off,
-                    double* fpart, std::uint32_t* fcnt, std::uint64_t* foff, Scalars* sc,
-                    std::uint32_t* ticket)
+hipError_t step_dev(hipStream_t s, std::size_t n_cap, internal::DevLoop* loop, int q,
+                    const double* est, double* err0, double* err1, const double* pest,
+                    double epsrel, int relerr, std::uint8_t* active, double* part,
+                    std::uint32_t* cnt, std::uint64_t* off, std::uint64_t* foff, Scalars* sc)
 {
   // one workgroup more than num_chunks(n_cap): a paired list may have one
   // chunk more than a flat one
   hipLaunchKernelGGL(k_step_dev, dim3(static_cast<unsigned>(num_chunks(n_cap) + 1)), dim3(kThreads),
-                     0, s, loop, est, err0, err1, pest, epsrel, relerr, active, part, cnt, off,
-                     fpart, fcnt, foff, sc, ticket);
+                     0, s, loop, q, est, err0, err1, pest, epsrel, relerr, active, part, cnt, off,
+                     foff, sc);
   return hipGetLastError();
 }
 

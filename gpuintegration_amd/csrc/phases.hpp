@@ -117,11 +117,11 @@ hipError_t to_levels(hipStream_t s, int d, std::size_t n, const double* H, const
 // Device-resident loop variants (lists of at most kDevLoopMax regions):
 // fixed launch shapes for n_cap regions, the actual count and selections
 // read from the descriptors; a descriptor with run == 0 makes them no-ops.
-hipError_t step_dev(hipStream_t s, std::size_t n_cap, internal::DevLoop* loop, const double* est,
-                    double* err0, double* err1, const double* pest, double epsrel, int relerr,
-                    std::uint8_t* active, double* part, std::uint32_t* cnt, std::uint64_t* off,
-                    double* fpart, std::uint32_t* fcnt, std::uint64_t* foff, Scalars* sc,
-                    std::uint32_t* ticket);
+// step_dev is the round's q-th step: it reads its[q] and writes its[q + 1].
+hipError_t step_dev(hipStream_t s, std::size_t n_cap, internal::DevLoop* loop, int q,
+                    const double* est, double* err0, double* err1, const double* pest,
+                    double epsrel, int relerr, std::uint8_t* active, double* part,
+                    std::uint32_t* cnt, std::uint64_t* off, std::uint64_t* foff, Scalars* sc);
 hipError_t compact_dev(hipStream_t s, std::size_t n_cap, const DevCompact* cp, int d,
                        double* L0, double* H0, double* L1, double* H1, std::uint8_t* P0,
                        std::uint8_t* P1, const std::uint8_t* active, const double* est,

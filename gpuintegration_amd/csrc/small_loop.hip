@@ -55,22 +55,6 @@ struct SmallShared {
   std::uint16_t src[kSmallMax];
 };
 
-// Four sums over a wave at once: the steps of ph::wave_reduce, interleaved.
-__device__ __forceinline__ void wave_reduce4(DD (&v)[4])
-{
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    DD o[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      o[i].hi = __shfl_xor(v[i].hi, off, 64);
-      o[i].lo = __shfl_xor(v[i].lo, off, 64);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = ph::dd_add(v[i], o[i]);
-  }
-}
-
 template <int D, class F>
 __global__ void __launch_bounds__(kSmallThreads)
     k_small_loop(F f, DevLoop* __restrict__ loop, int iterations, const SmallBufs b,
@@ -172,7 +156,7 @@ __global__ void __launch_bounds__(kSmallThreads)
         const std::uint32_t c = static_cast<std::uint32_t>(__popcll(__ballot(a)));
         if (lane == 0) sh.cnt[chunk][k][cwave] = c;
       }
-      wave_reduce4(v);
+      ph::wave_reduce4(v);
       if (lane == 0)
 #pragma unroll
         for (int i = 0; i < 4; ++i) sh.sums[i][wave] = v[i];

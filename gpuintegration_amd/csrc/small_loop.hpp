@@ -14,7 +14,7 @@ namespace internal {
 constexpr std::size_t kSmallMax = 2 * phases::kChunk;
 // Iterations per launch: the first launch of a segment, and later ones
 // (replayed from a graph); both fit the trace of a round.
-constexpr int kSmallFirst = 32, kSmallNext = 8;
+constexpr int kSmallFirst = 24, kSmallNext = 8;
 
 // The workspace's buffers the loop works in (those of the device-resident
 // loop), and the launch constants.

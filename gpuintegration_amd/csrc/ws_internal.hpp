@@ -46,6 +46,9 @@ struct TraceRec {
 // memory between rounds).  decide_step (devloop_decide.hpp, run by the last
 // workgroup of k_step_dev) makes the host loop's per-iteration decisions on
 // it; see integrate_impl for when the loop runs on the device.
+// Iterations queued per round at most: a round that stops early leaves the
+// rest as no-op launches, so the length trades round trips for those.
+constexpr int kDevQueueMax = 16;
 constexpr int kDevTrace = 64;  // trace records per round (a round is at most 64 iterations)
 enum : std::int32_t {
   kDevRun = 0,        // every queued iteration committed; more may follow
@@ -83,6 +86,10 @@ struct DevLoop {
   // k_step_dev's workgroup counter (zero between launches)
   std::uint32_t ticket;
   TraceRec trace[kDevTrace];
+  // the queued iterations of a round: entry q is what launch q of the round
+  // evaluates, refines and filters (entry 0 = it at the round's start, later
+  // ones written by the step before), so that it holds still while they read
+  pagani_dev_iter its[kDevQueueMax + 1];
 };
 
 // LoopState::relerr value of a run whose relerr flag follows the
