@@ -10,7 +10,6 @@ namespace mc {
 namespace {
 
 constexpr int kNd = PAGANI_MC_BINS;
-constexpr double kAlpha = 1.5;  // Internal_Vegas_Params alph, vegas_utils.cuh:158
 
 // rebin (vegasT.cuh:617-637) on one axis: xi[0..nd] with xi[0] = 0, weights
 // r[1..nd]; the new right edges put rc of the weight in every bin, linear
@@ -69,57 +68,6 @@ void grid_init(int ndim, double* xi)
     rebin(1 / static_cast<double>(kNd), kNd, r, xin, x);
     x[0] = 0.0;
   }
-}
-
-void refine(int ndim, int hist_dims, double* hist, double* xi)
-{
-  const double xnd = kNd;
-  double r[kNd + 1], xin[kNd + 1];
-  for (int j = 0; j < hist_dims; ++j) {
-    double* h = hist + static_cast<std::size_t>(j) * kNd - 1;  // bins h[1..kNd]
-    double xo = h[1], xn = h[2], rc, dt;
-    h[1] = (xo + xn) / 2.0;
-    dt = h[1];
-    for (int i = 2; i < kNd; ++i) {
-      rc = xo + xn;
-      xo = xn;
-      xn = h[i + 1];
-      h[i] = (rc + xn) / 3.0;
-      dt += h[i];
-    }
-    h[kNd] = (xo + xn) / 2.0;
-    dt += h[kNd];
-    if (dt > 0.0) {
-      rc = 0.0;
-      for (int i = 1; i <= kNd; ++i) {
-        r[i] = std::pow((1.0 - h[i] / dt) / (std::log(dt) - std::log(h[i])), kAlpha);
-        rc += r[i];
-      }
-      rebin(rc / xnd, kNd, r, xin, xi + static_cast<std::size_t>(j) * (kNd + 1));
-    }
-  }
-  if (hist_dims == 1)
-    for (int j = 1; j < ndim; ++j)
-      for (int i = 1; i <= kNd; ++i) xi[static_cast<std::size_t>(j) * (kNd + 1) + i] = xi[i];
-}
-
-void combine(double ti, double tsi, int iteration, double& si, double& schi, double& swgt,
-             double& estimate, double& chi_sq, double& errorest)
-{
-  const double wgt = 1.0 / tsi;
-  si += wgt * ti;
-  schi += wgt * ti * ti;
-  swgt += wgt;
-  estimate = si / swgt;
-  chi_sq = (schi - si * estimate) / (static_cast<double>(iteration) - 0.9999);
-  if (chi_sq < 0.0) chi_sq = 0.0;
-  errorest = std::sqrt(1.0 / swgt);
-}
-
-int get_status(double estimate, double errorest, int iteration, double epsrel, double epsabs)
-{
-  const bool ok = std::fabs(errorest / estimate) <= epsrel || errorest <= epsabs;
-  return (ok && iteration >= 5) ? 0 : 1;
 }
 
 bool adjust_params(double& ncall, int& total_iters)

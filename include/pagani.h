@@ -603,7 +603,9 @@ typedef struct pagani_mc_result {
  * fb and f2b to part[2g], part[2g+1] and its bin histograms to
  * hist[g*hist_dims*PAGANI_MC_BINS ...]. */
 typedef struct pagani_mc_args {
-  const double* xi; /* device grid, ndim x (PAGANI_MC_BINS+1) */
+  const double* xi; /* device grid, ndim x (PAGANI_MC_BINS+1), and one entry
+                     * more: not zero when the run has ended, and this queued
+                     * iteration samples nothing */
   double lo[PAGANI_MC_MAX_DIM];
   double dx[PAGANI_MC_MAX_DIM];
   double xjac, dxg, xnd;

@@ -145,7 +145,9 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(F f, pagani_mc_args a)
   const int tid = threadIdx.x;
   for (int i = tid; i < D * (kBins + 1); i += kThreads) sxi[i] = a.xi[i];
   for (int i = tid; i < hd * kBins; i += kThreads) shist[i] = 0.0;
+  const double ended = a.xi[D * (kBins + 1)];
   __syncthreads();
+  if (ended != 0.0) return;  // the run ended before this queued iteration
 
   // Thread g of the grid (wave W = g / 64, lane l) takes chunk
   // l * (T / 64) + W of the T chunks: the lanes of a wave work in cubes far
