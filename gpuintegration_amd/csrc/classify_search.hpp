@@ -10,8 +10,8 @@
 // kTreeDepth moves away; search_replay then runs the reference's loop from
 // the start, reading measured states from the cache, until it finishes or
 // meets a state not measured yet.  Run to completion this way, the result
-// is that of the sequential loop.  The device runs the replay in one
-// workgroup (k_search), so the host enqueues probe passes without reading
+// is that of the sequential loop.  The device runs the replay in the
+// pass's last workgroup (k_multi_threshold_dev), so the host enqueues probe passes without reading
 // anything back; the host runs the same function when it searches itself.
 // Plain IEEE double without contraction on both sides, so both make the
 // same decisions.
@@ -185,6 +185,7 @@ __host__ __device__ inline void search_tree(double t, double low, double high, d
 struct SearchState {
   SearchInputs in;
   int pending;  // a probe pass of S is queued (its results go to the cache)
+  std::uint32_t ticket;  // its workgroups that are through (zero between passes)
   int len;      // cache entries
   std::uint64_t passes;
   SearchStep step;

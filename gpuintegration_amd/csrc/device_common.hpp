@@ -81,6 +81,31 @@ __device__ __forceinline__ void block_reduce4(DD (&v)[4], DD (&sh)[4][kThreads /
   }
 }
 
+// Records that the workgroup finishing last reads in the same launch: stored
+// and loaded at agent scope, which is where every XCD sees them, and counted
+// by a ticket taken when the stores have arrived there.  A release fence
+// would also write back everything else in the XCD's L2.
+__device__ __forceinline__ void store_agent(double* p, double v)
+{
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double load_agent(const double* p)
+{
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The calling wave's stores have arrived.
+__device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// The workgroup's place in the order of finishing, one lane of the wave that
+// stored its record.
+__device__ __forceinline__ std::uint32_t take_ticket(std::uint32_t* ticket)
+{
+  wait_stores();
+  const std::uint32_t t =
+      __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  asm volatile("" ::: "memory");
+  return t;
+}
+
 // Reduce a DD over a 256-thread block; every thread gets the result.
 __device__ __forceinline__ DD block_reduce(DD v, DD* sh)
 {

@@ -205,7 +205,7 @@ int classify(pagani_ws* ws, Classifier& c, const double* err, std::size_t n, dou
     HIP_TRY(ws, ph::search_start(ws->stream, ws->d_search, ws->d_scal, in));
     for (;;) {
       for (int r = 0; r < kSearchRounds; ++r)
-        HIP_TRY(ws, ph::search_round(ws->stream, n, err, ws->d_search, ws->d_mpart, ws->d_mout));
+        HIP_TRY(ws, ph::search_round(ws->stream, n, err, ws->d_search, ws->d_mpart));
       HIP_TRY(ws, hipMemcpyAsync(ws->h_search, ws->d_search, sizeof(SearchState),
                                  hipMemcpyDeviceToHost, ws->stream));
       HIP_TRY(ws, hipStreamSynchronize(ws->stream));

@@ -270,8 +270,8 @@ __device__ __forceinline__ void multi_threshold_block(std::size_t n, const doubl
   __shared__ double ts[K];
   __shared__ double bsum[K - 1][kThreads];
   __shared__ std::uint32_t bcnt[K - 1][kThreads];
-  __shared__ DD sh[kThreads / 64];
-  __shared__ std::uint32_t shc[kThreads / 64];
+  __shared__ DD sh[K][kThreads / 64];
+  __shared__ std::uint32_t shc[K][kThreads / 64];
   const int tid = threadIdx.x;
   if (tid < K) ts[tid] = T.t[tid];
 #pragma unroll
@@ -305,22 +305,51 @@ __device__ __forceinline__ void multi_threshold_block(std::size_t n, const doubl
     for (int i = 0; i < kAhead; ++i) add(r[i]);
   }
   for (; t < n; t += stride) add(err[t]);
-  // suffix sums: candidate k counts the buckets k..K-2
+  // suffix sums: candidate k counts the buckets k..K-2; the workgroup's
+  // reductions of four candidates side by side (one after the other, fifteen
+  // took 12 us)
+  static_assert(K % 4 == 0, "candidates in fours");
   double* out = bpart + static_cast<std::size_t>(blockIdx.x) * 3 * kMaxThresholds;
+  const int lane = tid & 63, wave = tid >> 6;
   double sum = 0.0;
   std::uint32_t cnt = 0;
-  for (int k = K - 2; k >= 0; --k) {
-    sum += bsum[k][tid];
-    cnt += bcnt[k][tid];
-    if (k < T.k) {  // uniform
-      const DD s = block_reduce(DD{sum, 0.0}, sh);
-      const std::uint32_t c = block_count(cnt, shc);
-      if (tid == 0) {
-        out[3 * k] = s.hi;
-        out[3 * k + 1] = s.lo;
-        out[3 * k + 2] = static_cast<double>(c);
+  for (int k0 = K - 4; k0 >= 0; k0 -= 4) {
+    DD v[4];
+    std::uint32_t c[4];
+#pragma unroll
+    for (int i = 3; i >= 0; --i) {
+      if (k0 + i < K - 1) {
+        sum += bsum[k0 + i][tid];
+        cnt += bcnt[k0 + i][tid];
       }
+      v[i] = DD{sum, 0.0};
+      c[i] = cnt;
     }
+    if (k0 >= T.k) continue;  // uniform
+    wave_reduce4(v);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) c[i] += __shfl_xor(c[i], off, 64);
+    if (lane == 0)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        sh[k0 + i][wave] = v[i];
+        shc[k0 + i][wave] = c[i];
+      }
+  }
+  __syncthreads();
+  if (tid < T.k) {
+    DD s = sh[tid][0];
+    std::uint32_t c = shc[tid][0];
+#pragma unroll
+    for (int w = 1; w < kThreads / 64; ++w) {
+      s = dd_add(s, sh[tid][w]);
+      c += shc[tid][w];
+    }
+    store_agent(out + 3 * tid, s.hi);
+    store_agent(out + 3 * tid + 1, s.lo);
+    store_agent(out + 3 * tid + 2, static_cast<double>(c));
   }
 }
 
@@ -332,32 +361,28 @@ __global__ void __launch_bounds__(kThreads)
   multi_threshold_block<K>(n, err, T, bpart);
 }
 
-// The pass the device search queued (nothing when it queued none).
-template <int K>
-__global__ void __launch_bounds__(kThreads)
-    k_multi_threshold_dev(std::size_t n, const double* __restrict__ err,
-                          const internal::SearchState* __restrict__ st, double* __restrict__ bpart)
+// Fold the kMultiBlocks partials of candidate k: lane j of a wave folds
+// blocks j, j+64, j+128, ... in order, then a fixed butterfly over the wave.
+// All of a lane's loads are in flight together.
+__device__ __forceinline__ void multi_reduce_wave(int k, const double* bpart, double& count,
+                                                  double& sum)
 {
-  if (!st->pending) return;
-  // the candidates are read where they lie (a local copy of the set would
-  // go to scratch memory, thread by thread)
-  multi_threshold_block<K>(n, err, st->S, bpart);
-}
-
-// Fold the kMultiBlocks partials of k_multi_threshold: one wave per
-// threshold (workgroup k), lane j folds blocks j, j+64, j+128, ... in order,
-// then a fixed butterfly over the wave.
-__device__ __forceinline__ void multi_reduce_wave(int nblocks, int nthr,
-                                                  const double* __restrict__ bpart,
-                                                  double* __restrict__ out)
-{
-  const int k = blockIdx.x, j = threadIdx.x;
+  constexpr int kBlocks = kMultiBlocks / 64;
+  static_assert(kMultiBlocks % 64 == 0, "whole rounds of a wave");
+  const int j = threadIdx.x & 63;
+  double v[kBlocks][3];
+#pragma unroll
+  for (int i = 0; i < kBlocks; ++i)
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      v[i][q] = load_agent(bpart + static_cast<std::size_t>(i * 64 + j) * 3 * kMaxThresholds +
+                           3 * k + q);
   DD s{0.0, 0.0};
   double c = 0.0;  // counts are integers below 2^53: exact
-  for (int b = j; b < nblocks; b += 64) {
-    const double* p = bpart + static_cast<std::size_t>(b) * 3 * kMaxThresholds + 3 * k;
-    s = dd_add(s, DD{p[0], p[1]});
-    c += p[2];
+#pragma unroll
+  for (int i = 0; i < kBlocks; ++i) {
+    s = dd_add(s, DD{v[i][0], v[i][1]});
+    c += v[i][2];
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -367,57 +392,78 @@ __device__ __forceinline__ void multi_reduce_wave(int nblocks, int nthr,
     s = dd_add(s, o);
     c += __shfl_xor(c, off, 64);
   }
-  if (j == 0) {
-    out[k] = c;
-    out[nthr + k] = s.hi + s.lo;
+  count = c;
+  sum = s.hi + s.lo;
+}
+
+__global__ void __launch_bounds__(64)
+    k_multi_reduce(int nthr, const double* __restrict__ bpart, double* __restrict__ out)
+{
+  double c, s;
+  multi_reduce_wave(blockIdx.x, bpart, c, s);
+  if (threadIdx.x == 0) {
+    out[blockIdx.x] = c;
+    out[nthr + blockIdx.x] = s;
   }
 }
 
-__global__ void __launch_bounds__(64)
-    k_multi_reduce(int nblocks, int nthr, const double* __restrict__ bpart,
-                   double* __restrict__ out)
+// search_tree on a wave: lane i < kTreeNodes walks to node i from the root
+// (the moves are the bits of i + 1 below its first, most significant first:
+// 0 raises, 1 lowers) and ranks its key among the others', stable.
+__device__ __forceinline__ void search_tree_wave(double t, double low, double high,
+                                                 internal::SearchState* st)
 {
-  multi_reduce_wave(nblocks, nthr, bpart, out);
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x & 63;
+  double x = t, lo = low, hi = high;
+  for (int bit = 30 - __clz(lane + 1); bit >= 0; --bit) {
+    if (((lane + 1) >> bit) & 1) {
+      const double y = x - fabs(lo - x) * .5;
+      hi = x;
+      x = y;
+    } else {
+      const double y = x + fabs(hi - x) * .5;
+      lo = x;
+      x = y;
+    }
+  }
+  const double key = x != x ? HUGE_VAL : x;
+  int rank = 0;
+#pragma unroll
+  for (int j = 0; j < internal::kTreeNodes; ++j) {
+    const double other = __shfl(key, j, 64);
+    if (other < key || (other == key && j < lane)) ++rank;
+  }
+  if (lane < internal::kTreeNodes) {
+    st->node[lane] = x;
+    st->perm[rank] = lane;
+    st->S.t[rank] = key;
+  } else if (lane < kMaxThresholds) {
+    st->S.t[lane] = HUGE_VAL;
+  }
+  if (lane == 0) st->S.k = internal::kTreeNodes;
 }
 
-__global__ void __launch_bounds__(64)
-    k_multi_reduce_dev(int nblocks, const internal::SearchState* __restrict__ st,
-                       const double* __restrict__ bpart, double* __restrict__ out)
-{
-  if (!st->pending || static_cast<int>(blockIdx.x) >= st->S.k) return;
-  multi_reduce_wave(nblocks, st->S.k, bpart, out);
-}
-
-// The heuristic classifier's search on the device, one wave: first != 0
-// starts a search from `in` with the errors' min and max from the minmax
-// finalize (sc); otherwise the last queued pass's results (mout) join the
-// measured states.  Then search_replay runs the reference's loop over them
-// (every lane the same scalar work, the lookups spread over the lanes) and
-// either records the result or queues the next pass.  A search that would
-// outgrow the cache or the step limit stops with step.overflow set, for the
-// host to finish.
-__global__ void __launch_bounds__(64)
-    k_search(internal::SearchState* __restrict__ st, const Scalars* __restrict__ sc,
-             const double* __restrict__ mout, int first, internal::SearchInputs in)
+// The heuristic classifier's search on the device, one wave: First starts a
+// search from `in`; otherwise the last pass's results (mcnt, msum,
+// by candidate slot) join the measured states.  Then search_replay runs the
+// reference's loop over them (every lane the same scalar work, the lookups
+// spread over the lanes) and either records the result or queues the next
+// pass.  A search that would outgrow the cache or the step limit stops with
+// step.overflow set, for the host to finish.
+template <bool First>
+__device__ __forceinline__ void search_wave(internal::SearchState* st,
+                                            const internal::SearchInputs& in, const double* mcnt,
+                                            const double* msum)
 {
   namespace I = internal;
-  const int lane = threadIdx.x;
-  int len = 0;
-  bool fresh = false;  // the last pass's results, read from mout
-  if (first) {
-    in.mn = sc->mn;
-    in.mx = sc->mx;
-  } else {
-    if (!st->pending) return;
-    in = st->in;
-    len = st->len;
-    fresh = true;
-  }
-  // measured states: the cache of earlier launches, then the last pass
-  // (slot i of the pass holds tree node perm[i]).  Each lane holds its share
-  // of the states in registers (entry q*64 + lane, NaN where there is none,
-  // which equals nothing, as a NaN state equals nothing), so a lookup is a
-  // few compares and ballots; only a hit reads memory.
+  const int lane = threadIdx.x & 63;
+  int len = First ? 0 : st->len;
+  // measured states: the cache of earlier passes, then the last pass (slot i
+  // of the pass holds tree node perm[i]).  Each lane holds its share of the
+  // states in registers (entry q*64 + lane, NaN where there is none, which
+  // equals nothing, as a NaN state equals nothing), so a lookup is a few
+  // compares and ballots; only a hit reads memory.
   static_assert(I::kSearchCache <= 4 * 64, "four cache entries per lane");
   double cv[4];
 #pragma unroll
@@ -425,8 +471,10 @@ __global__ void __launch_bounds__(64)
     const int i = q * 64 + lane;
     cv[q] = i < len ? st->ct[i] : __builtin_nan("");
   }
-  const double fv =
-      fresh && lane < I::kTreeNodes ? st->node[st->perm[lane]] : __builtin_nan("");
+  const bool slot = lane < I::kTreeNodes;
+  double fv = __builtin_nan("");
+  if constexpr (!First)
+    if (slot) fv = st->node[st->perm[lane]];
   auto find = [&](double x, std::uint64_t& c, double& d) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -438,41 +486,91 @@ __global__ void __launch_bounds__(64)
         return true;
       }
     }
-    const unsigned long long hit = __ballot(fv == x);
-    if (hit) {
-      const int slot = __ffsll(static_cast<long long>(hit)) - 1;
-      c = static_cast<std::uint64_t>(mout[slot]);
-      d = mout[st->S.k + slot];
-      return true;
+    if constexpr (!First) {
+      const unsigned long long hit = __ballot(fv == x);
+      if (hit) {
+        const int k = __ffsll(static_cast<long long>(hit)) - 1;
+        c = static_cast<std::uint64_t>(mcnt[k]);
+        d = msum[k];
+        return true;
+      }
     }
     return false;
   };
   I::SearchStep step;
   I::search_replay(in, find, step);
-  // every lane has read what it needs: the state may change now
-  __syncthreads();
+  // every lane has read what it needs (one wave, in step): the state may
+  // change now, an entry per lane
+  if constexpr (!First) {
+    if (slot) {
+      st->ct[len + lane] = fv;
+      st->ccnt[len + lane] = static_cast<std::uint64_t>(mcnt[lane]);
+      st->cdot[len + lane] = msum[lane];
+    }
+    len += I::kTreeNodes;
+  }
+  if (!step.done && !step.overflow && len + I::kTreeNodes > I::kSearchCache) step.overflow = 1;
+  const bool next = !step.done && !step.overflow;
+  if (next) search_tree_wave(step.t, step.low, step.high, st);
   if (lane == 0) {
-    if (first) {
+    if constexpr (First) {
       st->in = in;
       st->passes = 0;
-    }
-    if (fresh) {
-      for (int i = 0; i < I::kTreeNodes; ++i) {
-        st->ct[len + i] = st->node[st->perm[i]];
-        st->ccnt[len + i] = static_cast<std::uint64_t>(mout[i]);
-        st->cdot[len + i] = mout[st->S.k + i];
-      }
-      len += I::kTreeNodes;
+      st->ticket = 0;
     }
     st->len = len;
-    st->pending = 0;
-    if (!step.done && !step.overflow && len + I::kTreeNodes > I::kSearchCache) step.overflow = 1;
     st->step = step;
-    if (!step.done && !step.overflow) {
-      I::search_tree(step.t, step.low, step.high, st->node, st->S, st->perm);
-      st->pending = 1;
-      st->passes += 1;
+    st->pending = next ? 1 : 0;
+    if (next) st->passes = (First ? 0 : st->passes) + 1;
+  }
+}
+
+// Starts a search: the errors' min and max from the minmax finalize (sc).
+__global__ void __launch_bounds__(64)
+    k_search(internal::SearchState* __restrict__ st, const Scalars* __restrict__ sc,
+             internal::SearchInputs in)
+{
+  in.mn = sc->mn;
+  in.mx = sc->mx;
+  search_wave<true>(st, in, nullptr, nullptr);
+}
+
+// The pass the device search queued (nothing when it queued none), and in
+// the workgroup that finishes last the fold of its partials and the search's
+// next step.  As three launches a pass of 4 10^6 errors took 35 + 11 + 6..33
+// us and three more no-ops for every pass not needed.
+template <int K>
+__global__ void __launch_bounds__(kThreads)
+    k_multi_threshold_dev(std::size_t n, const double* __restrict__ err, internal::SearchState* st,
+                          double* bpart)
+{
+  __shared__ double mcnt[K], msum[K];
+  __shared__ int last;
+  if (!st->pending) return;
+  // the candidates are read where they lie (a local copy of the set would
+  // go to scratch memory, thread by thread)
+  multi_threshold_block<K>(n, err, st->S, bpart);
+  // the first wave stored the partials: its own stores, then the ticket
+  if (threadIdx.x < 64) {
+    const bool mine = threadIdx.x == 0;
+    wait_stores();
+    if (mine) last = take_ticket(&st->ticket) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int k = wave; k < st->S.k; k += kThreads / 64) {
+    double c, s;
+    multi_reduce_wave(k, bpart, c, s);
+    if (lane == 0) {
+      mcnt[k] = c;
+      msum[k] = s;
     }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    if (lane == 0) st->ticket = 0;
+    search_wave<false>(st, st->in, mcnt, msum);
   }
 }
 
@@ -659,7 +757,7 @@ __device__ __forceinline__ void finalize_block(std::size_t nchunks, const double
                                                Scalars* __restrict__ out, int with_minmax)
 {
   __shared__ std::uint64_t wtot[kFinThreads / 64];
-  __shared__ DD tree[kFinThreads];
+  __shared__ DD tree[4][kFinThreads];
   __shared__ double tmn[kFinThreads], tmx[kFinThreads];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   DD s[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
@@ -698,30 +796,24 @@ __device__ __forceinline__ void finalize_block(std::size_t nchunks, const double
       __syncthreads();
     }
   }
+  // the sums' trees side by side: eight barriers, not eight per sum
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    tree[tid] = s[i];
-    __syncthreads();
-    for (int stride = kFinThreads / 2; stride > 0; stride >>= 1) {
-      if (tid < stride) tree[tid] = dd_add(tree[tid], tree[tid + stride]);
-      __syncthreads();
+  for (int i = 0; i < 4; ++i) tree[i][tid] = s[i];
+  tmn[tid] = mn;
+  tmx[tid] = mx;
+  __syncthreads();
+  for (int stride = kFinThreads / 2; stride > 0; stride >>= 1) {
+    if (tid < stride) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) tree[i][tid] = dd_add(tree[i][tid], tree[i][tid + stride]);
+      tmn[tid] = fmin(tmn[tid], tmn[tid + stride]);
+      tmx[tid] = fmax(tmx[tid], tmx[tid + stride]);
     }
-    if (tid == 0) out->sum[i] = tree[0].hi + tree[0].lo;
     __syncthreads();
-  }
-  if (with_minmax) {
-    tmn[tid] = mn;
-    tmx[tid] = mx;
-    __syncthreads();
-    for (int stride = kFinThreads / 2; stride > 0; stride >>= 1) {
-      if (tid < stride) {
-        tmn[tid] = fmin(tmn[tid], tmn[tid + stride]);
-        tmx[tid] = fmax(tmx[tid], tmx[tid + stride]);
-      }
-      __syncthreads();
-    }
   }
   if (tid == 0) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) out->sum[i] = tree[i][0].hi + tree[i][0].lo;
     out->count = running;
     out->mn = with_minmax ? tmn[0] : 0.0;
     out->mx = with_minmax ? tmx[0] : 0.0;
@@ -753,15 +845,6 @@ __global__ void __launch_bounds__(kFinThreads)
 // carries the chunk's errors and flags (needed by later launches only).  The
 // loop's state is copied to LDS and back by all lanes, so that the decisions,
 // one lane's, wait for no memory.
-__device__ __forceinline__ void store_agent(double* p, double v)
-{
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ double load_agent(const double* p)
-{
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 __global__ void __launch_bounds__(kThreads)
     k_step_dev(internal::DevLoop* __restrict__ loop, int q, const double* __restrict__ est,
                double* err0, double* err1, const double* __restrict__ pest, double epsrel,
@@ -802,11 +885,7 @@ __global__ void __launch_bounds__(kThreads)
       store_agent(p + 2 * i + 1, v[i].lo);
     }
     __hip_atomic_store(cnt + chunk, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // the stores above have reached memory before the ticket is taken
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    last = __hip_atomic_fetch_add(&loop->ticket, 1u, __ATOMIC_RELAXED,
-                                  __HIP_MEMORY_SCOPE_AGENT) == nch - 1;
-    asm volatile("" ::: "memory");
+    last = take_ticket(&loop->ticket) == nch - 1;
   }
   __syncthreads();
   if (!last) return;
@@ -1266,22 +1345,15 @@ hipError_t threshold_flags(hipStream_t s, std::size_t n, const double* est, cons
 hipError_t search_start(hipStream_t s, internal::SearchState* st, const Scalars* sc,
                         const internal::SearchInputs& in)
 {
-  hipLaunchKernelGGL(k_search, dim3(1), dim3(64), 0, s, st, sc, nullptr, 1, in);
+  hipLaunchKernelGGL(k_search, dim3(1), dim3(64), 0, s, st, sc, in);
   return hipGetLastError();
 }
 
 hipError_t search_round(hipStream_t s, std::size_t n, const double* err,
-                        internal::SearchState* st, double* bpart, double* mout)
+                        internal::SearchState* st, double* bpart)
 {
   hipLaunchKernelGGL(k_multi_threshold_dev<kMaxThresholds>, dim3(kMultiBlocks), dim3(kThreads), 0,
                      s, n, err, st, bpart);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_multi_reduce_dev, dim3(kMaxThresholds - 1), dim3(64), 0, s, kMultiBlocks,
-                     st, bpart, mout);
-  if ((e = hipGetLastError()) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_search, dim3(1), dim3(64), 0, s, st, nullptr, mout, 0,
-                     internal::SearchInputs{});
   return hipGetLastError();
 }
 
@@ -1297,7 +1369,7 @@ hipError_t multi_threshold(hipStream_t s, std::size_t n, const double* err, cons
                      n, err, U, bpart);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_multi_reduce, dim3(T.k), dim3(64), 0, s, kMultiBlocks, T.k, bpart, out);
+  hipLaunchKernelGGL(k_multi_reduce, dim3(T.k), dim3(64), 0, s, T.k, bpart, out);
   return hipGetLastError();
 }
 

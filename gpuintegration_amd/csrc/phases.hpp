@@ -166,13 +166,13 @@ hipError_t threshold_flags(hipStream_t s, std::size_t n, const double* est, cons
 // The heuristic classifier's threshold search on the device
 // (classify_search.hpp): search_start begins a search from `in` with the
 // errors' min and max from the last minmax finalize (sc) and queues its first
-// probe pass; each search_round runs the queued pass over err (bpart,
-// mout: the multi-threshold scratch) and the replay that queues the next
-// one.  Rounds after the search has finished do nothing.
+// probe pass; each search_round is one launch that runs the queued pass over
+// err (bpart: the multi-threshold scratch) and the replay that queues the
+// next one.  Rounds after the search has finished do nothing.
 hipError_t search_start(hipStream_t s, internal::SearchState* st, const Scalars* sc,
                         const internal::SearchInputs& in);
 hipError_t search_round(hipStream_t s, std::size_t n, const double* err,
-                        internal::SearchState* st, double* bpart, double* mout);
+                        internal::SearchState* st, double* bpart);
 
 hipError_t multi_threshold(hipStream_t s, std::size_t n, const double* err,
                            const ThresholdSet& T, double* bpart, double* out);
