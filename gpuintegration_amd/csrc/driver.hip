@@ -372,7 +372,18 @@ struct LoopVars {
   bool has_parents;
   pagani_result* cum;
   Classifier* clf;
+  std::size_t* unformed;  // the uniform split whose list is not formed yet, 0 when it is
 };
+
+// Form the run's first list, k^ndim equal regions, if it is not yet.
+int form_list(pagani_ws* ws, std::size_t n, std::size_t& k)
+{
+  if (k)
+    HIP_TRY(ws, ph::uniform_split(ws->stream, ws->ndim, k, n, ws->L[ws->cur].p, ws->H[ws->cur].p,
+                                  ws->lv.on != 0));
+  k = 0;
+  return PAGANI_OK;
+}
 
 // Run iterations on the device, with one host round trip per round, until
 // the device loop stops.  A round over a short list of an FP64 Genz integrand
@@ -396,7 +407,7 @@ int run_device_segment(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double eps
   // the live list (its own bounds, or its parents' and their halved axes)
   // and the parents' estimates are kept; everything else is sized for the
   // capacity
-  const std::size_t rows = ws->split ? v.n / 2 : v.n;
+  const std::size_t rows = *v.unformed ? 0 : ws->split ? v.n / 2 : v.n;
   if ((rc = grow_keep(ws, ws->L[cur], cap * d, rows * d, "region bounds")) ||
       (rc = grow_keep(ws, ws->H[cur], cap * d, rows * d, "region bounds")) ||
       (rc = grow_keep(ws, ws->pdim[cur], cap / 2, ws->split ? rows : 0, "split axes")) ||
@@ -508,12 +519,14 @@ int run_device_segment(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double eps
     if (h.it.n <= scap) {
       // the loop's state is read from and written back to h_loop itself
       const int iterations = smalls ? kSmallNext : kSmallFirst;
+      const int split = static_cast<int>(*v.unformed);  // the first launch forms the list
+      *v.unformed = 0;
       h.any_slices = 1;
       h.round_cap = scap;
       if (ws->timing) record(ws, EV_DEV0);
       rc = launch(ws->graphs && smalls, scap, 0, [&]() -> int {
-        HIP_TRY(ws, launch_small_loop(ws->stream, genz->g, ws->h_loop, iterations, sb,
-                                      args.consts));
+        HIP_TRY(ws, launch_small_loop(ws->stream, genz->g, ws->h_loop, iterations, split,
+                                      sb, args.consts));
         return PAGANI_OK;
       });
       if (rc) return rc;
@@ -521,6 +534,7 @@ int run_device_segment(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double eps
       if (ws->timing) record(ws, EV_DEV1);
       HIP_TRY(ws, hipStreamSynchronize(ws->stream));
     } else {
+      if ((rc = form_list(ws, v.n, *v.unformed))) return rc;
       // A round's launches have as many waves per workgroup as its first
       // iteration's slice count, and grids for the largest list with that
       // slice count that a few iterations can lead to (an iteration at most
@@ -656,7 +670,7 @@ int integrate_impl(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double epsrel,
   harvest_compact(ws);
 
   // initial region list
-  std::size_t n = 0;
+  std::size_t n = 0, unformed = 0;
   if (resume) {
     n = st.n;
     ws->split = st.split != 0;
@@ -691,8 +705,7 @@ int integrate_impl(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double epsrel,
     }
     if ((rc = ensure(ws, ws->L[ws->cur], n * d, "region bounds"))) return rc;
     if ((rc = ensure(ws, ws->H[ws->cur], n * d, "region bounds"))) return rc;
-    HIP_TRY(ws, ph::uniform_split(ws->stream, d, k, n, ws->L[ws->cur].p, ws->H[ws->cur].p,
-                                  ws->lv.on != 0));
+    unformed = k;
   }
 
   const std::size_t total = st.mem_total;
@@ -721,6 +734,7 @@ int integrate_impl(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double epsrel,
   for (; it < 700 && n > 0; it++) {
     ws->scal_minmax = false;  // d_scal's min / max belong to an earlier list
     if (ws->iter_limit && iters_this_call == ws->iter_limit) {
+      if ((rc = form_list(ws, n, unformed))) return rc;
       st.it = it;
       st.n = n;
       st.has_parents = has_parents ? 1 : 0;
@@ -747,7 +761,7 @@ int integrate_impl(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double epsrel,
     if (ws->device_loop && !ws->iter_limit && ws->snapshot_iter == ~std::uint64_t(0) &&
         relerr != kRelerrPredictSplit && rec.level() == 0 &&
         n <= ph::kDevLoopMax && mem_ratio(n, d, total, mem_model) <= .1) {
-      LoopVars v{it, n, has_parents, &cum, &clf};
+      LoopVars v{it, n, has_parents, &cum, &clf, &unformed};
       DevOutcome outcome;
       if ((rc = run_device_segment(ws, eval, ctx, epsrel, epsabs, relerr, user_regions, lows,
                                    highs, v, outcome)))
@@ -763,6 +777,7 @@ int integrate_impl(pagani_ws* ws, pagani_eval_fn eval, void* ctx, double epsrel,
       reduced = true;
     }
     if (!reduced) {
+      if ((rc = form_list(ws, n, unformed))) return rc;
       iters_this_call++;
       if ((rc = ensure(ws, ws->est, n, "estimates")) || (rc = ensure(ws, ws->err0, n, "errors")) ||
           (rc = ensure(ws, ws->err1, n, "errors")) || (rc = ensure(ws, ws->dim, n, "split axes")) ||

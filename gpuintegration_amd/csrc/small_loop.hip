@@ -57,7 +57,7 @@ struct SmallShared {
 
 template <int D, class F>
 __global__ void __launch_bounds__(kSmallThreads)
-    k_small_loop(F f, DevLoop* __restrict__ loop, int iterations, const SmallBufs b,
+    k_small_loop(F f, DevLoop* __restrict__ loop, int iterations, int split, const SmallBufs b,
                  const pagani_eval_consts C)
 {
 #pragma clang fp contract(off)
@@ -76,6 +76,25 @@ __global__ void __launch_bounds__(kSmallThreads)
   if constexpr (kTab > 0)
     if (C.levels) detail::fill_pair_tables<D>(f, C, tab, tid, kSmallThreads);
   __syncthreads();
+  if (split) {
+    // the run's first list, split^D equal regions, as k_uniform_split forms it
+    const double len = 1. / static_cast<double>(split);
+    const int n = static_cast<int>(sh.s.it.n), cur = sh.s.it.cur ? 1 : 0;
+    for (int t = tid; t < n; t += kSmallThreads) {
+      int q = t;
+      for (int j = 0; j < D; ++j) {
+        const int id = q % split;
+        q /= split;
+        const std::size_t o = static_cast<std::size_t>(j) * n + t;
+        b.L[cur][o] = static_cast<double>(id) * len;
+        if (C.levels)
+          reinterpret_cast<std::uint16_t*>(b.H[cur])[o] = 0;
+        else
+          b.H[cur][o] = len;
+      }
+    }
+    __syncthreads();
+  }
 
   for (int iter = 0; iter < iterations && sh.s.it.run; ++iter) {
     const std::size_t n = sh.s.it.n;
@@ -254,18 +273,19 @@ int with_part_dim(int d, Fn&& fn)
 
 template <int Part>
 int launch_small_part(hipStream_t s, const pagani_genz& g, DevLoop* loop, int iterations,
-                      const SmallBufs& b, const pagani_eval_consts& C);
+                      int split, const SmallBufs& b, const pagani_eval_consts& C);
 
 template <>
 int launch_small_part<PAGANI_PART>(hipStream_t s, const pagani_genz& g, DevLoop* loop,
-                                   int iterations, const SmallBufs& b, const pagani_eval_consts& C)
+                                   int iterations, int split, const SmallBufs& b,
+                                   const pagani_eval_consts& C)
 {
   return with_part_dim<kPartFirst[PAGANI_PART]>(g.ndim, [&](auto D) {
     constexpr int Dv = decltype(D)::value;
     return visit_genz<double, Dv>(&g, [&](const auto& f) {
       using F = std::decay_t<decltype(f)>;
       hipLaunchKernelGGL((k_small_loop<Dv, F>), dim3(1), dim3(kSmallThreads), 0, s, f, loop,
-                         iterations, b, C);
+                         iterations, split, b, C);
       return hipGetLastError() == hipSuccess ? PAGANI_OK : PAGANI_EHIP;
     });
   });
@@ -287,14 +307,14 @@ std::size_t small_cap(int family, int d)
 }
 
 hipError_t launch_small_loop(hipStream_t s, const pagani_genz& g, DevLoop* loop, int iterations,
-                             const SmallBufs& b, const pagani_eval_consts& C)
+                             int split, const SmallBufs& b, const pagani_eval_consts& C)
 {
   const int d = g.ndim;
   auto launch = d < kPartFirst[1]   ? &launch_small_part<0>
                 : d < kPartFirst[2] ? &launch_small_part<1>
                 : d < kPartFirst[3] ? &launch_small_part<2>
                                     : &launch_small_part<3>;
-  return launch(s, g, loop, iterations, b, C) == PAGANI_OK ? hipSuccess : hipErrorLaunchFailure;
+  return launch(s, g, loop, iterations, split, b, C) == PAGANI_OK ? hipSuccess : hipErrorLaunchFailure;
 }
 #endif
 

@@ -33,8 +33,10 @@ std::size_t small_cap(int family, int d);
 
 // One launch: at most `iterations` iterations of the loop whose state is at
 // `loop` (pinned host memory, read at the start and written back at the end).
+// split > 0: the list is the run's first, split^ndim equal regions, not
+// formed yet.
 hipError_t launch_small_loop(hipStream_t s, const pagani_genz& g, DevLoop* loop, int iterations,
-                             const SmallBufs& b, const pagani_eval_consts& C);
+                             int split, const SmallBufs& b, const pagani_eval_consts& C);
 
 }  // namespace internal
 }  // namespace pagani
