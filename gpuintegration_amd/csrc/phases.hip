@@ -844,7 +844,10 @@ __global__ void __launch_bounds__(kFinThreads)
 // nothing else replaces a release, whose write-back of the whole L2 also
 // carries the chunk's errors and flags (needed by later launches only).  The
 // loop's state is copied to LDS and back by all lanes, so that the decisions,
-// one lane's, wait for no memory.
+// one lane's, wait for no memory.  With a ticket and a fence for every
+// workgroup of the grid and the decisions in memory a step took 17 us on two
+// workgroups and 35-45 us on a grid of 257; per integral, then -> now: 3D
+// Gaussian at 1e-4 267 -> 228 us, 6D corner peak at 1e-6 1.52 -> 1.12 ms.
 __global__ void __launch_bounds__(kThreads)
     k_step_dev(internal::DevLoop* __restrict__ loop, int q, const double* __restrict__ est,
                double* err0, double* err1, const double* __restrict__ pest, double epsrel,

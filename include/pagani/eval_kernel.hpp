@@ -1514,11 +1514,17 @@ template <class F>
 constexpr int kPairWaves = detail::is_masked<F>::value ? 4 : 8;
 template <class F>
 constexpr int kPairPerSimd = detail::is_masked<F>::value ? 3 : 4;
-// tiles from which a level-form list takes pair_kernel
+// tiles from which a level-form list takes pair_kernel: 512 workgroups, two a
+// CU, so that forming the tables overlaps another workgroup's evaluation; a
+// shorter list's time is one region's latency chain, which the tables'
+// barrier would lengthen
 constexpr std::size_t kPairLong = 4096;
 
 // Kernel: the evaluation of a has_pair_sums integrand on a level-form list at
-// one wave per tile of 64 regions (slices == 1), with its tables.
+// one wave per tile of 64 regions (slices == 1), with its tables.  Bound by
+// vector issue (8D Gaussian, 31.5 M regions: 1 592 instructions a region, 88 %
+// of the issue rate; 1.45 ms a launch against 2.15-2.22 for the factored sums
+// with two factors per axis and magnitude).
 template <int D, class F>
 __global__ void __launch_bounds__(64 * kPairWaves<F>, kPairPerSimd<F>)
     pair_kernel(F f, const pagani_dev_iter* __restrict__ it, std::size_t n_arg,
