@@ -144,7 +144,7 @@ __device__ void run_item(const F& f0, const SegItem& it, const SegPtrs& p, std::
       const std::size_t t = live ? t0 : n - 1;
       constexpr bool kPairs = detail::has_pair_sums<F>::value;
       detail::LoadedRow<kPairs ? D : 1> row(p.L[cur], p.H[cur], nullptr, n, t, C);
-      detail::eval_regions_wave<D, F, double, kPairs>(
+      detail::eval_regions_wave<D, F, double, kPairs, true>(
           f, p.L[cur], p.H[cur], nullptr, n, t, live, C.lows, C.range, C.jac, C, 1, 0, lane,
           nullptr, &row, nullptr, p.est, p.err0, p.dim);
     }

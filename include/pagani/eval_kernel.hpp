@@ -799,18 +799,14 @@ __device__ __forceinline__ float cos_real(float x) { return ::cosf(x); }
 // Returns false, having done nothing, when an angle could leave the range of
 // the FP64 sine and cosine (math::kTrigRange).
 template <int D, class F, class Real>
-__device__ __forceinline__ bool cosine_sums(F& f, const double (&cR)[D], const double (&hR)[D],
-                                            double jac, const pagani_eval_consts& C,
+__device__ __forceinline__ bool cosine_sums(F& f, double phi0, const double (&hR)[D], double jac,
+                                            const pagani_eval_consts& C,
                                             double (&rs)[PAGANI_NRULES], int& bisect)
 {
 #pragma clang fp contract(off)
-  double phi0 = f.phase_angle();
   double hmax = 0.0;
 #pragma unroll
-  for (int j = 0; j < D; ++j) {
-    phi0 += cR[j];
-    hmax = __builtin_fmax(hmax, __builtin_fabs(hR[j]));
-  }
+  for (int j = 0; j < D; ++j) hmax = __builtin_fmax(hmax, __builtin_fabs(hR[j]));
   // every lambda is below 1: the axis angles are at most |h_j|
   if (!(__builtin_fabs(phi0) <= math::kTrigRange && hmax <= math::kTrigRange)) return false;
   Real sr, cr;
@@ -959,13 +955,19 @@ __device__ __forceinline__ double scaled(double x, double a) { return x * a; }
 // Region setup, Phases.cuh:323-349: volume, widest axis, and the centre /
 // width of region t in the integrand's frame (user coordinates, moved to the
 // origin and scaled for a centred integrand); a rule point is x = c - g w.
-template <int D, class F>
+// A cosine integrand's angle at the centre is summed on the way: FusedAngle
+// adds each axis as one FMA of the unscaled centre, else the scaled centre is
+// added.  The two differ in the last bit, which a smooth integrand's null-rule
+// sums (cancelled to 1e-8 .. 1e-11 of their terms) show in the fourth digit
+// of an error or later, so each kernel keeps to one of them: the batch's segment
+// kernel to the first, the launches and the short-list loop to the second.
+template <int D, bool FusedAngle = false, class F>
 __device__ __forceinline__ void region_frame(F& f, const double* __restrict__ L,
                                              const double* __restrict__ H,
                                              const std::uint8_t* __restrict__ pdim, std::size_t n,
                                              std::size_t t, const pagani_eval_consts& C,
                                              double (&cR)[D], double (&hR)[D], double& vol,
-                                             int& maxdim)
+                                             int& maxdim, double& angle)
 {
 #pragma clang fp contract(off)
   const double* lows = C.lows;
@@ -973,6 +975,8 @@ __device__ __forceinline__ void region_frame(F& f, const double* __restrict__ L,
   double maxr = 0.0;
   vol = 1.0;
   maxdim = 0;
+  constexpr bool kAngle = is_cosine<F>::value && has_origin<F>::value && has_axis_scale<F>::value;
+  if constexpr (kAngle) angle = f.phase_angle();
   LoadedRow<D> row(L, H, pdim, n, t, C);
 #pragma unroll
   for (int j = 0; j < D; ++j) {
@@ -992,8 +996,11 @@ __device__ __forceinline__ void region_frame(F& f, const double* __restrict__ L,
     hR[j] = r * range[j];
     if constexpr (has_origin<F>::value) cR[j] -= f.origin(j);
     if constexpr (has_origin<F>::value && has_axis_scale<F>::value) {
+      if constexpr (kAngle && FusedAngle)
+        angle = __builtin_fma(cR[j], f.axis_scale(j), angle);
       cR[j] = scaled(cR[j], f.axis_scale(j));
       hR[j] = scaled(hR[j], f.axis_scale(j));
+      if constexpr (kAngle && !FusedAngle) angle += cR[j];
     }
   }
 }
@@ -1239,7 +1246,7 @@ __device__ __forceinline__ double point_generator(const pagani_eval_consts& C, i
 // == 1); with more than one, every wave of the workgroup passes one barrier,
 // and only wave 0 returns true (holding the results).  `lows`, `range`,
 // `jac` describe the integration box.
-template <int D, class F, class Real, bool Pairs>
+template <int D, class F, class Real, bool Pairs, bool FusedAngle>
 __device__ __forceinline__ bool eval_region_values(
     F& f, const double* __restrict__ L, const double* __restrict__ H,
     const std::uint8_t* __restrict__ pdim, std::size_t n, std::size_t t,
@@ -1252,7 +1259,7 @@ __device__ __forceinline__ bool eval_region_values(
   double rs[PAGANI_NRULES] = {0.0, 0.0, 0.0, 0.0, 0.0};
   int bisect = 0;
   bool done = false;
-  double cR[D], hR[D];
+  double cR[D], hR[D], angle = 0.0;
   if constexpr (Pairs)
     done = pair_region<D, F>(f, *row, L, H, lows, range, C, tab, rs, bisect, vol);
   if (!done) {
@@ -1260,14 +1267,14 @@ __device__ __forceinline__ bool eval_region_values(
     // takes the generic loop after them: the compiler must not see that the
     // two share values
     if constexpr (Pairs) asm volatile("" : "+v"(t));
-    region_frame<D>(f, L, H, pdim, n, t, C, cR, hR, vol, bisect);
+    region_frame<D, FusedAngle>(f, L, H, pdim, n, t, C, cR, hR, vol, bisect, angle);
   }
   if constexpr (has_group_sums<F>::value) {
     done = group_sums<D, F>(f, cR, hR, C, slices, wave, rs, bisect);
   } else if constexpr (has_pair_sums<F>::value) {
     // a region out of the pair sums' range, and several waves: the generic loop
   } else if constexpr (is_cosine<F>::value && has_origin<F>::value && has_axis_scale<F>::value) {
-    if (slices == 1) done = cosine_sums<D, F, Real>(f, cR, hR, jac, C, rs, bisect);
+    if (slices == 1) done = cosine_sums<D, F, Real>(f, angle, hR, jac, C, rs, bisect);
   } else if constexpr (is_separable<F>::value) {
     if (slices == 1) done = separable_sums<D, F>(f, cR, hR, jac, C, rs, bisect);
   }
@@ -1383,7 +1390,7 @@ __device__ __forceinline__ bool eval_region_values(
 }
 
 // eval_region_values, stored: region t's estimate, error and split axis.
-template <int D, class F, class Real, bool Pairs>
+template <int D, class F, class Real, bool Pairs, bool FusedAngle = false>
 __device__ __forceinline__ void eval_regions_wave(
     F& f, const double* __restrict__ L, const double* __restrict__ H,
     const std::uint8_t* __restrict__ pdim, std::size_t n, std::size_t t, bool live,
@@ -1393,8 +1400,9 @@ __device__ __forceinline__ void eval_regions_wave(
 {
   double avg, er;
   int axis;
-  if (!eval_region_values<D, F, Real, Pairs>(f, L, H, pdim, n, t, lows, range, jac, C, slices, wave,
-                                      lane, part, row, tab, avg, er, axis))
+  if (!eval_region_values<D, F, Real, Pairs, FusedAngle>(f, L, H, pdim, n, t, lows, range, jac, C,
+                                                         slices, wave, lane, part, row, tab, avg,
+                                                         er, axis))
     return;
   if (live) {
     est[t] = avg;
@@ -1575,9 +1583,9 @@ __global__ void __launch_bounds__(256)
   const std::size_t t = i / F_;
   if (t >= n) return;
   const int p = static_cast<int>(i % F_);
-  double cR[D], hR[D], vol;
+  double cR[D], hR[D], vol, angle;
   int maxdim;
-  detail::region_frame<D>(f, L, H, P, n, t, C, cR, hR, vol, maxdim);
+  detail::region_frame<D>(f, L, H, P, n, t, C, cR, hR, vol, maxdim, angle);
   Real x[D];
 #pragma unroll
   for (int j = 0; j < D; ++j)
