@@ -1337,7 +1337,7 @@ __device__ __forceinline__ bool eval_region_values(
       }
 #pragma unroll
       for (int r = 0; r < PAGANI_NRULES; ++r)
-        rs[r] = __builtin_fma(C.w[2][r], s2, __builtin_fma(C.w[1][r], s1, C.w[0][r] * f0));
+        rs[r] = __builtin_fma(C.w[2][r], s2, __builtin_fma(C.w[0][r], f0, C.w[1][r] * s1));
     }
 
     // Sets 3..8 from the generator table, this wave's slice of the points.

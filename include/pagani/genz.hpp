@@ -69,10 +69,14 @@ __device__ __forceinline__ double fabs_(double x) { return __builtin_fabs(x); }
 __device__ __forceinline__ float fabs_(float x) { return __builtin_fabsf(x); }
 __device__ __forceinline__ double fmax_(double x, double y) { return __builtin_fmax(x, y); }
 __device__ __forceinline__ float fmax_(float x, float y) { return __builtin_fmaxf(x, y); }
-// written out where a sum is contracted, so that every kernel an integrand
-// is inlined into forms the same bits
+// x y + z.  FP64: the contraction written out, so that every kernel an
+// integrand is inlined into (the launches, the short-list loop, the segments)
+// forms the same bits.  FP32 integrands run in the evaluation kernel alone,
+// which contracts each place as it did before the others existed (the first
+// two products either way round, by how often they are used): 1 ulp of an FP32
+// value is 1e-3 of a small error estimate.
 __device__ __forceinline__ double fma_(double x, double y, double z) { return __builtin_fma(x, y, z); }
-__device__ __forceinline__ float fma_(float x, float y, float z) { return __builtin_fmaf(x, y, z); }
+__device__ __forceinline__ float fma_(float x, float y, float z) { return z + x * y; }
 }  // namespace math
 
 // The rule's generator magnitudes lambda1..lambda5 (rule.cpp's kLam): the
