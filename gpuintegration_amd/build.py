@@ -69,8 +69,8 @@ SLICE_BUCKETS = 32
 def generate_tuning_table():
     """Write the autotuner's measurements (tuning/eval_slices.json, from
     gpuintegration_amd/tune.py) as the C table driver.hip compiles in:
-    kTunedSlices[family][ndim][precision][size class], 0 where nothing was
-    measured."""
+    kTunedSlices[family][ndim][precision][size class], 0 where the rule of
+    choose_slices_n decides."""
     import json
     table = {}
     if os.path.exists(TUNING_JSON):
@@ -83,6 +83,12 @@ def generate_tuning_table():
             vals = [0] * SLICE_BUCKETS
             for b, s in row["slices"].items():
                 vals[int(b)] = int(s)
+            # lists of less than a batch: the smallest measured class's entry
+            # for the integrands evaluated by pair or group sums; the others'
+            # errors are rounding noise that another wave count would move
+            if p == 0 and row["family"] != "oscillatory":
+                first = min(int(b) for b in row["slices"])
+                vals[:first] = [vals[first]] * first
             table[(fam, d, p)] = vals
     lines = ["// generated by gpuintegration_amd/build.py from tuning/eval_slices.json",
              "static const std::uint8_t kTunedSlices[7][%d][2][%d] = {" % (MAX_DIM + 1,

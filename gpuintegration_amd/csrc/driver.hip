@@ -300,9 +300,9 @@ std::uint64_t round_cap(const pagani_ws* ws, std::uint64_t n, std::uint64_t cap,
   if (ws->slices_override <= 0)
     if (const std::uint8_t* t = tuned_table(ws)) {
       int b = slice_bucket(n);
-      const int e = tuned_entry(t, b);
+      const int e = t[b];
       if (e > 0) {
-        while (b + 1 < kSliceBuckets && tuned_entry(t, b + 1) == e &&
+        while (b + 1 < kSliceBuckets && t[b + 1] == e &&
                (std::uint64_t(1) << (b + 1)) <= cap)
           ++b;
         const std::uint64_t end = b + 1 < 64 ? (std::uint64_t(2) << b) - 1 : cap;

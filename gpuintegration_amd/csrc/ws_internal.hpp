@@ -29,7 +29,6 @@ namespace ph = pagani::phases;
 // tune.py per integrand family, dimension and precision; 0 = no
 // measurement (choose_slices_n's rule decides).
 constexpr int kSliceBuckets = 32;
-constexpr int kFirstTuned = 6;  // the smallest class measured
 
 template <class T>
 struct DevBuf {
@@ -398,14 +397,6 @@ __host__ __device__ inline int slice_bucket(std::size_t n)
   return b;
 }
 
-// The tuned table's entry for a size class, 0 where it has none; the classes
-// below the first measured one (lists of less than a batch) take that one's.
-__host__ __device__ inline int tuned_entry(const std::uint8_t* table, int b)
-{
-  while (b < kFirstTuned && table[b] == 0) ++b;
-  return table[b];
-}
-
 // Waves per batch of 64 regions for an n-region evaluation: the tuned
 // table's entry for n's size class when there is one; otherwise more waves
 // share a batch while there are too few batches to give every CU four
@@ -418,7 +409,7 @@ __host__ __device__ inline int choose_slices_n(std::size_t n, int num_cus, int o
 {
   if (override_ > 0) return override_ < PAGANI_MAX_SLICES ? override_ : PAGANI_MAX_SLICES;
   if (table) {
-    const int t = tuned_entry(table, slice_bucket(n));
+    const int t = table[slice_bucket(n)];
     if (t > 0) return t < PAGANI_MAX_SLICES ? t : PAGANI_MAX_SLICES;
   }
   const std::size_t batches = (n + 63) / 64;

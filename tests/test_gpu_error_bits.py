@@ -5,7 +5,8 @@ and an FP32 integrand's to the rounding of its values, so one more or one less
 contraction anywhere in an evaluation changes the errors a caller sees in
 their fifth digit or before.  Each route of these integrands has one order of
 operations: the segment kernel, the launches at one wave per batch and at
-several, the generic loop of FP32 integrands.  The values are that order's, bit for bit.
+several, the first list of less than a batch, the generic loop of FP32
+integrands.  The values are that order's, bit for bit.
 """
 import math
 
@@ -32,6 +33,13 @@ def segments(pg, d):
     assert codes == [0, 0] and b.stats()["segment_integrals"] == 2
     b.close()
     return [r.errorest.hex() for r in results]
+
+
+def short_list(pg, d):
+    """errorest of an oscillatory integral of one short list"""
+    with pg.Workspace(d, 0) as ws:
+        r = ws.integrate_genz("oscillatory", *_params("oscillatory", d), epsrel=1e-2, epsabs=1e-20)
+    return [r.errorest.hex()]
 
 
 def evaluated(pg, fam, d, precision, slices):
@@ -62,6 +70,15 @@ SEGMENTS = {
     6: ["0x1.5599b5dc1981fp-27", "0x1.5599b5dc1981fp-27"],
     8: ["0x1.feadc98cffedep-26", "0x1.feadc98cffedep-26"],
     10: ["0x1.23458138c747dp-24", "0x1.23458138c747dp-24"],
+}
+SHORT = {
+    2: ["0x1.021ce7e53caa0p-40"],
+    3: ["0x1.a1770f762eb0cp-37"],
+    4: ["0x1.0d586714c5d28p-35"],
+    5: ["0x1.7e58e08563950p-31"],
+    6: ["0x1.5599b5dcc1411p-27"],
+    8: ["0x1.feadc98cffedep-26"],
+    10: ["0x1.23458138ca926p-24"],
 }
 EVAL = {
     ("c0", 32, 1): {
@@ -154,6 +171,11 @@ EVAL = {
 @pytest.mark.parametrize("d", DIMS)
 def test_oscillatory_segments(pg, gpu, d):
     assert segments(pg, d) == SEGMENTS[d]
+
+
+@pytest.mark.parametrize("d", DIMS)
+def test_oscillatory_short_list(pg, gpu, d):
+    assert short_list(pg, d) == SHORT[d]
 
 
 @pytest.mark.parametrize("fam,precision,slices", EVALS)
