@@ -267,6 +267,9 @@ _SIGS = {
     "pagani_mc_integrate_cb": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_double, ctypes.c_double,
                                               _dp, _dp, ctypes.POINTER(McParams),
                                               ctypes.POINTER(McResult)]),
+    "pagani_mc_integrate_queued": (ctypes.c_int, [_vp, _vp, _vp, ctypes.c_double, ctypes.c_double,
+                                                  _dp, _dp, ctypes.POINTER(McParams),
+                                                  ctypes.POINTER(McResult)]),
     "pagani_mc_integrate_genz": (ctypes.c_int, [_vp, ctypes.POINTER(_Genz), ctypes.c_double,
                                                 ctypes.c_double, _dp, _dp,
                                                 ctypes.POINTER(McParams),

@@ -43,7 +43,7 @@ constexpr int kQueue = 16;
 
 // The run's state, doubles that follow the grid's ndim * (kBins + 1) entries.
 enum : int {
-  kEnded = 0,  // the run has ended (read by the sampling kernel)
+  kEnded = 0,  // the run has ended (pagani_mc_args::ended)
   kLive,       // this iteration was sampled: k_mc_step's order to run
   kSi,
   kSchi,
@@ -325,6 +325,7 @@ void fill_args(pagani_mc* mc, const pagani::mc::Setup& s, const Launch& l, int g
   a.part = mc->d_part;
   a.hist = mc->d_hist;
   a.stream = mc->stream;
+  a.ended = nullptr;
 }
 
 // One sampling launch and its reduction into d_out, queued.
@@ -370,13 +371,12 @@ int upload_grid(pagani_mc* mc, const double* xi, const pagani_mc_result* so_far)
 }
 
 // One vegas() run: adjust_iters iterations that refine the grid, then the
-// others up to titer.  Whole chunks of iterations are queued, each three
+// others up to titer.  Chunks of `queue` iterations are queued, each three
 // launches with no word from the host in between; when the stopping rule
-// ends the run, the rest of the chunk does nothing.  With timing on, a chunk
-// is one iteration.
-int run(pagani_mc* mc, pagani_mc_sample_fn sample, void* ctx, double epsrel, double epsabs,
-        const double* lows, const double* highs, const pagani_mc_params& p, double ncall,
-        int titer, pagani_mc_result* out)
+// ends the run, the rest of the chunk does nothing.
+int run(pagani_mc* mc, pagani_mc_sample_fn sample, void* ctx, int queue, double epsrel,
+        double epsabs, const double* lows, const double* highs, const pagani_mc_params& p,
+        double ncall, int titer, pagani_mc_result* out)
 {
   const int d = mc->ndim;
   pagani::mc::Setup s;
@@ -393,9 +393,10 @@ int run(pagani_mc* mc, pagani_mc_sample_fn sample, void* ctx, double epsrel, dou
   if ((rc = upload_grid(mc, xi.data(), out))) return rc;
   double* const state = mc->d_xi + xi.size();
   const double* const st = mc->h_xi + xi.size();
+  if (queue > 1) a.ended = state + kEnded;
   const int last = std::max(p.adjust_iters, titer);
   for (int it = 1; it <= last && out->status;) {
-    const int first = it, end = std::min(last, it + (mc->timing ? 1 : kQueue) - 1);
+    const int first = it, end = std::min(last, it + queue - 1);
     for (; it <= end; ++it) {
       const bool adjusts = it <= p.adjust_iters;
       a.hist_dims = adjusts ? static_cast<std::uint32_t>(hd) : 0;
@@ -468,6 +469,37 @@ pagani_mc_sample_fn genz_sampler(int ndim)
     case 8: return &genz_sample<8>;
     default: return nullptr;
   }
+}
+
+int integrate(pagani_mc* mc, pagani_mc_sample_fn sample, void* ctx, int queue, double epsrel,
+              double epsabs, const double* lows, const double* highs,
+              const pagani_mc_params* params, pagani_mc_result* out)
+{
+  if (!mc) return PAGANI_EBADARG;
+  if (!out || !sample) return fail(mc, PAGANI_EBADARG, "null argument");
+  std::memset(out, 0, sizeof(*out));
+  out->status = 1;
+  int rc = validate(mc, params, lows, highs);
+  if (rc) return rc;
+  MC_TRY(mc, hipSetDevice(mc->device));
+  const auto t0 = std::chrono::steady_clock::now();
+  mc->ti.clear();
+  mc->tsi.clear();
+  double ncall = params->ncall;
+  int titer = params->total_iters;
+  do {
+    out->runs++;
+    out->ncall = ncall;
+    rc = run(mc, sample, ctx, queue, epsrel, epsabs, lows, highs, *params, ncall, titer, out);
+    if (rc) {
+      out->status = 1;
+      return rc;
+    }
+  } while (params->adjust_params && out->status == 1 && pagani::mc::adjust_params(ncall, titer));
+  mc->stats.integrals++;
+  mc->stats.wall_ms +=
+      std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+  return PAGANI_OK;
 }
 
 }  // namespace
@@ -573,31 +605,17 @@ int pagani_mc_integrate_cb(pagani_mc* mc, pagani_mc_sample_fn sample, void* ctx,
                            double epsabs, const double* lows, const double* highs,
                            const pagani_mc_params* params, pagani_mc_result* out)
 {
-  if (!mc) return PAGANI_EBADARG;
-  if (!out || !sample) return fail(mc, PAGANI_EBADARG, "null argument");
-  std::memset(out, 0, sizeof(*out));
-  out->status = 1;
-  int rc = validate(mc, params, lows, highs);
-  if (rc) return rc;
-  MC_TRY(mc, hipSetDevice(mc->device));
-  const auto t0 = std::chrono::steady_clock::now();
-  mc->ti.clear();
-  mc->tsi.clear();
-  double ncall = params->ncall;
-  int titer = params->total_iters;
-  do {
-    out->runs++;
-    out->ncall = ncall;
-    rc = run(mc, sample, ctx, epsrel, epsabs, lows, highs, *params, ncall, titer, out);
-    if (rc) {
-      out->status = 1;
-      return rc;
-    }
-  } while (params->adjust_params && out->status == 1 && pagani::mc::adjust_params(ncall, titer));
-  mc->stats.integrals++;
-  mc->stats.wall_ms +=
-      std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-  return PAGANI_OK;
+  return integrate(mc, sample, ctx, 1, epsrel, epsabs, lows, highs, params, out);
+}
+
+int pagani_mc_integrate_queued(pagani_mc* mc, pagani_mc_sample_fn sample, void* ctx,
+                               double epsrel, double epsabs, const double* lows,
+                               const double* highs, const pagani_mc_params* params,
+                               pagani_mc_result* out)
+{
+  // with timing on, an event pair around each iteration's sampling
+  const int queue = mc && mc->timing ? 1 : kQueue;
+  return integrate(mc, sample, ctx, queue, epsrel, epsabs, lows, highs, params, out);
 }
 
 int pagani_mc_integrate_genz(pagani_mc* mc, const pagani_genz* f, double epsrel,
@@ -612,7 +630,7 @@ int pagani_mc_integrate_genz(pagani_mc* mc, const pagani_genz* f, double epsrel,
   if (f->family < PAGANI_GENZ_OSCILLATORY || f->family > PAGANI_GENZ_DISCONTINUOUS)
     return fail(mc, PAGANI_EBADARG, "unknown Genz family");
   pagani_genz g = *f;
-  return pagani_mc_integrate_cb(mc, fn, &g, epsrel, epsabs, lows, highs, params, out);
+  return pagani_mc_integrate_queued(mc, fn, &g, epsrel, epsabs, lows, highs, params, out);
 }
 
 int pagani_mc_trace(const pagani_mc* mc, double* ti, double* tsi, size_t cap, size_t* len)

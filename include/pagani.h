@@ -603,9 +603,7 @@ typedef struct pagani_mc_result {
  * fb and f2b to part[2g], part[2g+1] and its bin histograms to
  * hist[g*hist_dims*PAGANI_MC_BINS ...]. */
 typedef struct pagani_mc_args {
-  const double* xi; /* device grid, ndim x (PAGANI_MC_BINS+1), and one entry
-                     * more: not zero when the run has ended, and this queued
-                     * iteration samples nothing */
+  const double* xi; /* device grid, ndim x (PAGANI_MC_BINS+1) */
   double lo[PAGANI_MC_MAX_DIM];
   double dx[PAGANI_MC_MAX_DIM];
   double xjac, dxg, xnd;
@@ -620,6 +618,9 @@ typedef struct pagani_mc_args {
   double* part;
   double* hist;
   void* stream;       /* hipStream_t */
+  const double* ended; /* device flag of an iteration queued ahead: not zero when
+                        * the run has ended before it, and it samples nothing.
+                        * NULL: the iteration runs */
 } pagani_mc_args;
 
 /* A sampling callback launches the m-Cubes kernel for one integrand on
@@ -648,11 +649,20 @@ int pagani_mc_reset_stats(pagani_mc* mc);
 
 /* vegas() / integrate / simple_integrate (vegasT.cuh:640-1112) for any
  * integrand behind a sampling callback; lows/highs may be NULL (unit
- * cube).  Returns PAGANI_OK, or a negative code (then *out holds status 1). */
+ * cube).  The callback is called once per iteration of the run, with
+ * args->ended NULL.  Returns PAGANI_OK, or a negative code (then *out holds
+ * status 1). */
 int pagani_mc_integrate_cb(pagani_mc* mc, pagani_mc_sample_fn sample, void* ctx,
                            double epsrel, double epsabs, const double* lows,
                            const double* highs, const pagani_mc_params* params,
                            pagani_mc_result* out);
+/* The same for a callback whose launch does nothing where *args->ended is not
+ * zero (pagani::mc::sample_callback is one): iterations are queued up to 16 at
+ * a time, so it may be called up to 15 times past the run's last iteration. */
+int pagani_mc_integrate_queued(pagani_mc* mc, pagani_mc_sample_fn sample, void* ctx,
+                               double epsrel, double epsabs, const double* lows,
+                               const double* highs, const pagani_mc_params* params,
+                               pagani_mc_result* out);
 /* The same for a precompiled Genz integrand (ndim 2..8, FP64; m-Cubes'
  * precompiled samplers stop at 8 dimensions). */
 int pagani_mc_integrate_genz(pagani_mc* mc, const pagani_genz* f, double epsrel,

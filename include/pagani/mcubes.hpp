@@ -87,7 +87,7 @@ numint::integration_result run(IntegT const& integrand, double epsrel, double ep
   const quad::Volume<double, NDIM>* v = volume ? volume : &unit;
   pagani_mc_result r{};
   IntegT f = integrand;
-  const int rc = pagani_mc_integrate_cb(
+  const int rc = pagani_mc_integrate_queued(
       h.get(), &sample_callback<NDIM, IntegT, typename GeneratorType::stream>, &f, epsrel,
       epsabs, v->lows, v->highs, &p, &r);
   if (rc < 0) throw std::runtime_error(std::string("m-Cubes: ") + pagani_mc_last_error(h.get()));

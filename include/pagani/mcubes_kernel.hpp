@@ -143,11 +143,13 @@ __global__ void __launch_bounds__(kThreads) sample_kernel(F f, pagani_mc_args a)
   __shared__ double wsum[2][kThreads / 64];
   const int hd = static_cast<int>(a.hist_dims);
   const int tid = threadIdx.x;
+  // one load either way (of the grid's first edge without a flag), in flight
+  // with the grid's
+  const double flag = *(a.ended ? a.ended : a.xi);
   for (int i = tid; i < D * (kBins + 1); i += kThreads) sxi[i] = a.xi[i];
   for (int i = tid; i < hd * kBins; i += kThreads) shist[i] = 0.0;
-  const double ended = a.xi[D * (kBins + 1)];
   __syncthreads();
-  if (ended != 0.0) return;  // the run ended before this queued iteration
+  if (a.ended && flag != 0.0) return;  // the run ended before this queued iteration
 
   // Thread g of the grid (wave W = g / 64, lane l) takes chunk
   // l * (T / 64) + W of the T chunks: the lanes of a wave work in cubes far

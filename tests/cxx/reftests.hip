@@ -1056,6 +1056,61 @@ int mc_dispatch(const char* name, int mode, double epsrel, double ncall, int tit
 
 }  // namespace
 
+// A run whose callback counts its calls and passes on its own arguments, as a
+// program with a sampler of its own may: *calls and *out.
+extern "C" int reftest_mc_calls(double epsrel, double ncall, int titer, int itmax, int skip,
+                                int* calls, pagani_mc_result* out)
+{
+  struct Ctx {
+    Gauss1D f;
+    int calls;
+  } ctx{};
+  pagani_mc* mc = pagani_mc_create(1, -1);
+  if (!mc) return -1;
+  pagani_mc_params p{};
+  p.ncall = ncall;
+  p.total_iters = titer;
+  p.adjust_iters = itmax;
+  p.skip_iters = skip;
+  p.generator = PAGANI_MC_RNG_DEFAULT;
+  const int rc = pagani_mc_integrate_cb(
+      mc,
+      [](void* c, const pagani_mc_args* a) {
+        Ctx* x = static_cast<Ctx*>(c);
+        x->calls++;
+        return pagani::mc::launch<1, Gauss1D, pagani::mc::XoroStream>(x->f, a);
+      },
+      &ctx, epsrel, 1e-30, nullptr, nullptr, &p, out);
+  *calls = ctx.calls;
+  pagani_mc_destroy(mc);
+  return rc;
+}
+
+// One sampling launch over a program's own arguments: the grid xi (1D, device
+// memory of at least PAGANI_MC_BINS + 1 entries), `cubes` cubes of two points;
+// the sums of fb and f2b.
+extern "C" int reftest_mc_own_grid(const double* xi, unsigned cubes, double* part)
+{
+  double* d = nullptr;
+  if (hipMalloc(&d, 2 * sizeof(double)) != hipSuccess) return -1;
+  pagani_mc_args a{};
+  a.xi = xi;
+  a.dx[0] = 1.0;
+  a.ncubes = a.ng = cubes;
+  a.npg = 2;
+  a.cubes_per_thread = (cubes + pagani::mc::kThreads - 1) / pagani::mc::kThreads;
+  a.grid = 1;
+  a.xnd = PAGANI_MC_BINS;
+  a.dxg = a.xnd / cubes;
+  a.xjac = 1.0 / (2.0 * cubes);
+  a.key = 1;
+  a.part = d;
+  int rc = pagani::mc::launch<1, Gauss1D, pagani::mc::XoroStream>(Gauss1D{}, &a);
+  if (!rc && hipMemcpy(part, d, 2 * sizeof(double), hipMemcpyDeviceToHost) != hipSuccess) rc = -1;
+  (void)hipFree(d);
+  return rc;
+}
+
 // generator: 0 = Curand_generator (the library's default streams), 1 =
 // Custom_generator; mode: 0 integrate, 1 simple_integrate, 2 integrate1D,
 // 3 quad::mcubes, 4 cuda_mcubes::mcubes.

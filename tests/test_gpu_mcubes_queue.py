@@ -5,6 +5,9 @@ stopping rule ends inside a queue, before adjusting is over and after, with
 one grid for all axes; with timing on, the queue is one iteration long and the
 run the same.  Tolerances are those of the whole-run comparison with the
 oracle in test_gpu_mcubes.py."""
+import ctypes
+import os
+
 import numpy as np
 import pytest
 
@@ -50,3 +53,28 @@ def test_no_iterations():
                               ncall=1e4, total_iters=0, adjust_iters=0, skip_iters=0)
         assert (r["iters"], r["status"], r["neval"]) == (0, 1, 0)
         assert np.array_equal(mc.grid(), O.mc_grid_init(2))
+
+
+def _reftests():
+    return ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "cxx", "libreftests.so"))
+
+
+@pytest.mark.parametrize("eps,total,adjust,iters", [(1e-12, 20, 4, 20), (0.5, 40, 3, 5), (0.5, 40, 20, 5)])
+def test_callback_is_called_once_per_iteration(gpu, eps, total, adjust, iters):
+    """A callback need not know of iterations queued ahead: it sees the run's own, no more."""
+    calls, r = ctypes.c_int(), pg.McResult()
+    rc = _reftests().reftest_mc_calls(ctypes.c_double(eps), ctypes.c_double(2e4), total, adjust, 0,
+                                      ctypes.byref(calls), ctypes.byref(r))
+    assert (rc, r.iters, calls.value) == (0, iters, iters)
+
+
+def test_own_grid_ends_with_its_last_edge(gpu):
+    """A sampling launch over a program's own grid: what lies behind the ndim x
+    (PAGANI_MC_BINS + 1) edges does not decide whether it samples."""
+    import torch
+    edges = np.append(O.mc_grid_init(1).ravel(), 1.0)
+    xi = torch.from_numpy(edges).to(gpu)
+    part = (ctypes.c_double * 2)()
+    rc = _reftests().reftest_mc_own_grid(ctypes.c_void_p(xi.data_ptr()), 10000, part)
+    # the integral of exp(-50 (x - 0.3)^2) over [0, 1] from 2 points in each of 10^4 strata
+    assert rc == 0 and abs(part[0] - 0.25032445820538396) <= 1e-4 and part[1] > 0.0
