@@ -22,6 +22,7 @@
 
 #include "device_common.hpp"
 #include "genz_visit.hpp"
+#include "mcubes_edge.hpp"
 #include "mcubes_grid.hpp"
 #include "pagani.h"
 #include "pagani/mcubes_kernel.hpp"
@@ -198,17 +199,7 @@ __device__ bool refine_axis(const double* __restrict__ hist, const double* xi, d
   if (i < kBins) {
     const double rc = (total.hi + total.lo) / static_cast<double>(kBins);
     const double th = i * rc, tl = __builtin_fma(static_cast<double>(i), rc, -th);
-    int k = 1;  // the first bin whose prefix sum is not below i rc
-    for (int end = kBins; k < end;) {
-      const int mid = (k + end) / 2;
-      const ph::DD m = C[mid];
-      if (m.hi < th || (m.hi == th && m.lo < tl))
-        k = mid + 1;
-      else
-        end = mid;
-    }
-    const double dr = (C[k].hi - th) + (C[k].lo - tl);
-    edge = x[k] - (x[k] - x[k - 1]) * dr / r[k];
+    edge = pagani::mc::rebin_edge(C, r, x, kBins, th, tl);
   }
   return true;
 }

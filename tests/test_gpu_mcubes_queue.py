@@ -47,6 +47,20 @@ def test_queued_iterations_match_oracle(total, adjust, skip, eps, one_axis):
         _check(r, trace, xi, o)
 
 
+@pytest.mark.parametrize("generator", ["default", "lcg"])
+def test_empty_bins(generator):
+    """Nine tenths of axis 0's bins and half of axis 1's hold no weight."""
+    fam, a, u = "discontinuous", [5.0, 6.0], [0.1, 0.5]
+    with pg.MCubes(2) as mc:
+        r = mc.integrate_genz(fam, a, u, epsrel=1e-9, epsabs=1e-30, ncall=2e4, total_iters=8,
+                              adjust_iters=6, skip_iters=1, generator=generator, seed=9)
+        trace, xi = mc.trace(), mc.grid()
+    o = O.mc_integrate(fam, 2, O.params(a, u), 1e-9, 1e-30, 2e4, 8, 6, 1, generator, seed=9,
+                       trace_cap=64)
+    assert np.isfinite(xi).all()
+    _check(r, trace, xi, o)
+
+
 def test_no_iterations():
     with pg.MCubes(2) as mc:
         r = mc.integrate_genz("gaussian", [5.0, 5.0], [0.5, 0.5], epsrel=1e-3, epsabs=1e-30,

@@ -8,6 +8,8 @@ integrand, the inverse-CDF meaning of rebin) and statistically by the Genz
 closed forms.
 """
 import itertools
+import os
+import subprocess
 
 import numpy as np
 import pytest
@@ -223,3 +225,41 @@ def test_adjust_params_retries_with_ten_times_the_calls():
     assert r["runs"] >= 2
     assert r["ncall"] == 1e3 * 10 ** (r["runs"] - 1)
     assert r["status"] == 0
+
+EDGE_TEST = r"""
+#include "mcubes_edge.hpp"
+#include <cstdio>
+struct DD { double hi, lo; };
+int main()
+{
+  // weights 1 1 0 0 0 0 1 1 over unit bins; the empty run's prefix sums are 2
+  // to rounding, above and below in turn, and end below the sum looked for
+  const double u = 1e-32;
+  const double r[9] = {0, 1, 1, 0, 0, 0, 0, 1, 1}, x[9] = {0, 1, 2, 3, 4, 5, 6, 7, 8};
+  for (int s = 0; s < 81; ++s) {
+    double e[4];
+    for (int i = 0, q = s; i < 4; ++i, q /= 3) e[i] = u * (q % 3 - 1);
+    const DD C[9] = {{0, 0}, {1, 0}, {2, s % 2 ? 0.0 : -u}, {2, e[0]}, {2, e[1]},
+                     {2, e[2]}, {2, e[3]}, {3, 0}, {4, 0}};
+    std::printf("%.17g\n", pagani::mc::rebin_edge(C, r, x, 8, 2.0, 0.0));
+  }
+  const DD C[9] = {{0, 0}, {1, 0}, {2, 0}, {2, 0}, {2, 0}, {2, 0}, {2, 0}, {3, 0}, {4, 0}};
+  std::printf("%.17g %.17g %.17g\n", pagani::mc::rebin_edge(C, r, x, 8, 0.25, 0.0),
+              pagani::mc::rebin_edge(C, r, x, 8, 2.0, 1e-20), pagani::mc::rebin_edge(C, r, x, 8, 3.5, 0.0));
+}
+"""
+
+
+def test_refined_edge_on_a_run_of_empty_bins(tmp_path):
+    # the edge is where the weight is, at one end of the run or the other;
+    # a bin of weight zero is never divided by
+    src, exe = tmp_path / "edge.cpp", tmp_path / "edge"
+    src.write_text(EDGE_TEST)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    subprocess.run(["g++", "-std=c++17", "-Wno-unknown-pragmas", "-D__host__=", "-D__device__=",
+                    "-I", os.path.join(root, "gpuintegration_amd", "csrc"), str(src), "-o", str(exe)],
+                   check=True)
+    *ties, inside = subprocess.run([str(exe)], capture_output=True, text=True,
+                                   check=True).stdout.splitlines()
+    assert len(ties) == 81 and set(ties) <= {"2", "6"}
+    assert [float(v) for v in inside.split()] == [0.25, 6.0, 7.5]
