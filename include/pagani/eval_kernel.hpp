@@ -185,9 +185,10 @@ struct has_pair_sums<F, std::void_t<decltype(std::declval<const F&>().pair_sums(
     : std::true_type {};
 
 // Additive integrands (term, outer) may give outer summed over the points of
-// a group: `double sum2(s0, s1)`, `double sum4(s0, s1, s2, s3)`, with `bool
-// sum_safe(const double (&c)[D], const double (&h)[D])` true where every
-// point of a region with centre c and widths h may be summed so.
+// a group: `double sum1(b0)`, `sum2(b0, b1)`, `sum4(b0, b1, b2, b3)` of bases
+// b = base() + sum_j term(j, v_j), with `bool sum_safe(const double (&c)[D],
+// const double (&h)[D])` true where every point of a region with centre c and
+// widths h may be summed so.
 template <class F, class = void>
 struct has_group_sums : std::false_type {};
 template <class F>
@@ -666,13 +667,15 @@ __device__ __forceinline__ bool separable_sums(F& f, const double (&cR)[D], cons
 }
 
 // Rule sums and split axis of one region for an additive integrand with group
-// sums (has_group_sums): a point's value is outer of the centre's joined
-// terms plus the moved axes' changes, and the points of a set are taken in
-// groups of two and four.  The groups are dealt to the `slices` waves that
+// sums (has_group_sums): a point's base is the centre's plus the moved axes'
+// changes, and the points of a set are taken in groups of two and four.  The
+// centre's base is held with the rounding of its sum (E), which every point
+// adds to a change before the two are joined: left out, it would be an error
+// all points of a region share.  The groups are dealt to the `slices` waves that
 // share the batch in turn (uniformly, so a wave's loops hold scalars only);
 // wave 0 also takes sets 0-4, whose axis points give the fourth differences.
 // Without contraction, so every kernel that inlines this forms the same bits.
-// Bound by FP64 issue: 1 105 points at 8D, 10 instructions each.
+// Bound by FP64 issue: 1 105 points at 8D, 8 instructions each.
 template <int D, class F>
 __device__ __forceinline__ bool group_sums(F& f, const double (&cR)[D], const double (&hR)[D],
                                            const pagani_eval_consts& C, int slices, int wave,
@@ -680,11 +683,13 @@ __device__ __forceinline__ bool group_sums(F& f, const double (&cR)[D], const do
 {
 #pragma clang fp contract(off)
   if (!f.sum_safe(cR, hR)) return false;
-  double T0[D], S0;
+  double T0[D], S0 = f.base(), E = 0.0;
 #pragma unroll
   for (int j = 0; j < D; ++j) {
     T0[j] = f.term(j, cR[j]);
-    S0 = j ? S0 + T0[j] : T0[0];
+    const double s = S0 + T0[j], b = s - S0;
+    E += (S0 - (s - b)) + (T0[j] - b);
+    S0 = s;
   }
   auto change = [&](int j, double g) {
     return f.term(j, __builtin_fma(g, hR[j], cR[j])) - T0[j];
@@ -700,13 +705,13 @@ __device__ __forceinline__ bool group_sums(F& f, const double (&cR)[D], const do
   }
   if (wave == 0) {
     // sets 0-2 and the fourth differences, Sample.cuh:176-218, and sets 3-4
-    v[0] = f.outer(S0);
+    v[0] = f.sum1(S0 + E);
     const double base = v[0] * (2 * (1 - C.ratio));
     double maxdiff = 0.0;
 #pragma unroll
     for (int j = 0; j < D; ++j) {
-      const double fab = f.sum2(S0 + d1p[j], S0 + d1n[j]);
-      const double fcd = f.sum2(S0 + d2p[j], S0 + d2n[j]);
+      const double fab = f.sum2(S0 + (d1p[j] + E), S0 + (d1n[j] + E));
+      const double fcd = f.sum2(S0 + (d2p[j] + E), S0 + (d2n[j] + E));
       v[1] += fab;
       v[2] += fcd;
       const double diff = __builtin_fabs(__builtin_fma(C.ratio, fab, base) - fcd);
@@ -714,8 +719,8 @@ __device__ __forceinline__ bool group_sums(F& f, const double (&cR)[D], const do
         maxdiff = diff;
         bisect = j;
       }
-      v[3] += f.sum2(S0 + change(j, -C.lambda3), S0 + change(j, C.lambda3));
-      v[4] += f.sum2(S0 + change(j, -C.lambda4), S0 + change(j, C.lambda4));
+      v[3] += f.sum2(S0 + (change(j, -C.lambda3) + E), S0 + (change(j, C.lambda3) + E));
+      v[4] += f.sum2(S0 + (change(j, -C.lambda4) + E), S0 + (change(j, C.lambda4) + E));
     }
   }
   int turn = 0;  // the wave that takes the next group
@@ -727,7 +732,7 @@ __device__ __forceinline__ bool group_sums(F& f, const double (&cR)[D], const do
   // sets 5-7: (+-lambda1, +-lambda1), (+-lambda1, +-lambda2) and the triples
 #pragma unroll 1
   for (int j = 0; j < D; ++j) {
-    const double aj = S0 + d1p[j], bj = S0 + d1n[j];
+    const double aj = S0 + (d1p[j] + E), bj = S0 + (d1n[j] + E);
 #pragma unroll 1
     for (int k = 0; k < D; ++k) {
       if (k == j) continue;
@@ -768,7 +773,7 @@ __device__ __forceinline__ bool group_sums(F& f, const double (&cR)[D], const do
 #pragma unroll 1
     for (int hq = 0; hq < (1 << HB); ++hq) {
       if (!mine()) continue;
-      double hs = 0.0;
+      double hs = f.base();
 #pragma unroll
       for (int j = LB; j < D; ++j) hs += ((hq >> (j - LB)) & 1) ? tn[j] : tp[j];
 #pragma unroll

@@ -71,3 +71,69 @@ def test_corner_peak_groups(pg, gpu, d, slices, first):
     L = _boxes(rng, H)
     L[0, ::3] = 0.0
     _compare(pg, gpu, "corner_peak", a, [0.0] * d, L, H, slices)
+
+
+def _fma(x, y, z):
+    return (x.astype(np.longdouble) * y + z).astype(np.float64)
+
+
+def _point_by_point(pg, family, a, u, L, H):
+    """The rule's estimates of regions, every point of it by itself: in extended precision, in FP64 with the
+    kernel's centred points, and the sum of the terms' magnitudes."""
+    d, n = L.shape
+    k2 = 1.0  # the product peak's constant, as the descriptor's integrand holds it
+    for v in a:
+        k2 *= v * v
+    w, _, _, _, sb, _ = pg.rule_tables(d)
+    set_of = np.repeat(np.arange(9), np.diff(sb))
+    a, u = np.array(a)[:, None], np.array(u)[:, None]
+    x0, ld = (L + H / 2 - u if family == "product_peak" else L + H / 2) * a, np.longdouble
+    exact, scale, sums = np.zeros(n, ld), np.zeros(n, ld), np.zeros((9, n))
+    for p, s in enumerate(set_of):
+        g = np.array([pg.rule_point(d, p, j) for j in range(d)])[:, None]
+        x = (L.astype(ld) + H.astype(ld) / 2) - g.astype(ld) * H
+        v = _fma(-g, H * a, x0)
+        if family == "corner_peak":
+            fx = (1 + (a * x).sum(0)) ** -(d + 1)
+            b = np.ones(n)
+            for j in range(d):
+                b = b + v[j]
+            f, q = np.ones(n), b
+            for j in range(d):
+                q = q * b
+            f = 1.0 / q
+        else:
+            fx = ld(k2) / (1 + (a.astype(ld) * (x - u)) ** 2).prod(0)
+            q = np.ones(n)
+            for j in range(d):
+                q = q * _fma(v[j], v[j], 1.0)
+            f = k2 / q
+        exact += ld(w[s][0]) * fx
+        scale += abs(ld(w[s][0])) * fx
+        sums[s] += f
+    plain = np.zeros(n)
+    for s in range(9):
+        plain = _fma(np.full(n, w[s][0]), sums[s], plain)
+    return exact, plain, scale
+
+
+@pytest.mark.parametrize("family", ["corner_peak"])
+@pytest.mark.parametrize("d", [2, 3, 5])
+def test_rounding_is_that_of_single_points(pg, gpu, family, d):
+    """Sums over groups of points round no worse than the points one by one: the root mean square of the
+    regions' errors against extended precision, within 1.25 (a group's last roundings are shared by its
+    points, those of single points average out)."""
+    n = 20000 if d < 5 else 6000
+    rng = np.random.default_rng(40 + d)
+    a, u = genz_params(family, d, seed=3)
+    H = 0.5 ** rng.integers(1, 7, size=(d, n))
+    L = _boxes(rng, H)
+    exact, plain, scale = _point_by_point(pg, family, a, u, L, H)
+    rms = lambda est: float(np.sqrt((((est - exact) / scale) ** 2).mean()))  # noqa: E731
+    vol = H.prod(0)  # a power of two
+    with pg.Workspace(d, 0) as ws:
+        for slices in ((1, 4) if family == "corner_peak" else (1,)):
+            ws.set_slices(slices)
+            est = gpu_eval(ws, gpu, family, a, u, np.ascontiguousarray(L.ravel()),
+                           np.ascontiguousarray(H.ravel()), n)[0]
+            assert rms(est / vol) <= 1.25 * rms(plain)
