@@ -175,8 +175,8 @@ struct has_axis_aux<F, std::void_t<decltype(std::declval<const F&>().axis_aux(0,
 // `width_arg(int j, double h)`, the functions of the axis' width alone; table holds kTableSize doubles in LDS
 // (`fill_table(double*, int tid, int threads)`), or is NULL.  The nested type Centre
 // collects the axes' centres (add(f, j, c, h)), says whether the sums and
-// their products stay in range (safe(f)) and gives the centre's value up to
-// value() (value(f)).
+// their products stay in range (safe(f)) and gives the centre's value
+// (value(f)).
 template <class F, class = void>
 struct has_pair_sums : std::false_type {};
 template <class F>
@@ -1181,9 +1181,8 @@ __device__ __forceinline__ bool pair_region(F& f, LoadedRow<D>& row, const doubl
   }
   const double S0 = centre.value(f);
   const double v[PAGANI_NSETS] = {
-      f.value(kMasked && vmask ? 0.0 : S0),
-      f.value(S0 * g10), f.value(S0 * g01), f.value(S0 * acc3), f.value(S0 * acc4),
-      f.value(S0 * e2),  f.value(S0 * g11), f.value(S0 * e3),   f.value(S0 * prod)};
+      kMasked && vmask ? 0.0 : S0, S0 * g10, S0 * g01, S0 * acc3, S0 * acc4, S0 * e2,
+      S0 * g11, S0 * e3, S0 * prod};
   rule_sums(v, C, rs);
   if constexpr (kMasked) {
     // a masked integrand's factors are bounded only by the box: a region

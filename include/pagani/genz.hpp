@@ -304,7 +304,10 @@ struct ProductPeak {
   // factors are A/p and A/q, their sum A (p + q) / (p q).  The five
   // reciprocals of an axis come from one (the product of the five p q, then
   // unwound), so an axis has one division where the factors one by one have
-  // twenty.  |v|, |h| <= 1e7 keeps that product, and the centre's prod_j A,
+  // twenty.  The chain's rounding and that of the products is taken out of
+  // each quotient by its remainder: the sum rounds as two factors one by one
+  // do (without it a region's error is 1.1 to 1.2 times theirs, 2D to 5D; 7D,
+  // 200 003 regions: 25.5 -> 26.6 us).  |v|, |h| <= 1e7 keeps that product, and the centre's prod_j A,
   // below 1e150.
   struct Centre {
     double den = 1.0, big = 0.0;
@@ -314,7 +317,7 @@ struct ProductPeak {
       big = __builtin_fmax(big, __builtin_fmax(__builtin_fabs(c), __builtin_fabs(h)));
     }
     __device__ bool safe(const ProductPeak&) const { return big <= 1e7; }
-    __device__ double value(const ProductPeak&) const { return 1.0 / den; }
+    __device__ double value(const ProductPeak& f) const { return f.k2 / den; }
   };
   static constexpr int kWidthValues = 0, kTableSize = 0;
   template <class R = Real, if_double<R> = 0>
@@ -323,25 +326,27 @@ struct ProductPeak {
   {
 #pragma clang fp contract(off)
     const double A = __builtin_fma(v, v, 1.0);
-    double pq[5], left[5];  // the products p q, and the product of those before
+    double p[5], q[5], pq[5], left[5];  // the products p q, and the product of those before
     double run = 1.0;
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
       const double vp = __builtin_fma(kLambda[i], h, v), vm = __builtin_fma(-kLambda[i], h, v);
-      const double p = __builtin_fma(vp, vp, 1.0), q = __builtin_fma(vm, vm, 1.0);
-      s[i] = A * (p + q);
-      pq[i] = p * q;
+      p[i] = __builtin_fma(vp, vp, 1.0);
+      q[i] = __builtin_fma(vm, vm, 1.0);
+      pq[i] = p[i] * q[i];
       left[i] = run;
       run *= pq[i];
     }
-    double r = math::recip(run);
+    double r = __builtin_amdgcn_rcp(run);
+    r = __builtin_fma(r, __builtin_fma(-run, r, 1.0), r);
 #pragma unroll
     for (int i = 4; i >= 0; --i) {
-      s[i] *= r * left[i];
+      const double t = p[i] + q[i], num = A * t, ri = r * left[i], y = num * ri;
+      const double rem = __builtin_fma(-y, pq[i], num) + __builtin_fma(A, t, -num);
+      s[i] = __builtin_fma(__builtin_fma(-y, __builtin_fma(p[i], q[i], -pq[i]), rem), ri, y);
       r *= pq[i];
     }
   }
-  __device__ double value(double p) const { return outer(p); }
   static constexpr bool multiplicative = true;
   static constexpr bool linear_outer = true;
   __device__ double term(int, double v) const { return 1.0 / (1.0 + v * v); }
@@ -566,7 +571,6 @@ struct Gaussian {
       }
     }
   }
-  __device__ double value(double p) const { return p; }
 };
 
 // exp(-sum a_i |x_i - u_i|)
@@ -639,7 +643,6 @@ struct C0 {
       }
     }
   }
-  __device__ double value(double p) const { return p; }
   // outer(s + d) = outer(s) e^-d, non-negative terms (see Gaussian)
   static constexpr bool exponential = true;
   __device__ double factor(double d) const { return math::exp_factor(-d, Real()); }
@@ -743,7 +746,6 @@ struct Discontinuous {
       s[i] = (m ? w[2 * i] : 0.0) + (p ? w[2 * i + 1] : 0.0);
     }
   }
-  __device__ double value(double p) const { return p; }
   __device__ bool factor_safe(double s0) const
   {
     return __builtin_fabs(c + s0) <= kFactorRange<Real> - (sizeof(Real) == 8 ? 100.0 : 20.0);

@@ -117,7 +117,7 @@ def _point_by_point(pg, family, a, u, L, H):
     return exact, plain, scale
 
 
-@pytest.mark.parametrize("family", ["corner_peak"])
+@pytest.mark.parametrize("family", ["corner_peak", "product_peak"])
 @pytest.mark.parametrize("d", [2, 3, 5])
 def test_rounding_is_that_of_single_points(pg, gpu, family, d):
     """Sums over groups of points round no worse than the points one by one: the root mean square of the
