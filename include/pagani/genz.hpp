@@ -304,10 +304,11 @@ struct ProductPeak {
   // factors are A/p and A/q, their sum A (p + q) / (p q).  The five
   // reciprocals of an axis come from one (the product of the five p q, then
   // unwound), so an axis has one division where the factors one by one have
-  // twenty.  The chain's rounding and that of the products is taken out of
-  // each quotient by its remainder: the sum rounds as two factors one by one
-  // do (without it a region's error is 1.1 to 1.2 times theirs, 2D to 5D; 7D,
-  // 200 003 regions: 25.5 -> 26.6 us).  |v|, |h| <= 1e7 keeps that product, and the centre's prod_j A,
+  // twenty.  The chain's rounding and that of A (p + q) is taken out of each
+  // quotient by its remainder (not of lambda4's, which weighs in a null rule
+  // only): the sum rounds as two factors one by one do.  Without it a region's
+  // error is 1.1 to 1.2 times theirs, 2D to 5D; 8D, 10^6 regions: 54 -> 56 us,
+  // one by one 110.  |v|, |h| <= 1e7 keeps that product, and the centre's prod_j A,
   // below 1e150.
   struct Centre {
     double den = 1.0, big = 0.0;
@@ -343,7 +344,7 @@ struct ProductPeak {
     for (int i = 4; i >= 0; --i) {
       const double t = p[i] + q[i], num = A * t, ri = r * left[i], y = num * ri;
       const double rem = __builtin_fma(-y, pq[i], num) + __builtin_fma(A, t, -num);
-      s[i] = __builtin_fma(__builtin_fma(-y, __builtin_fma(p[i], q[i], -pq[i]), rem), ri, y);
+      s[i] = i == 3 ? y : __builtin_fma(rem, ri, y);
       r *= pq[i];
     }
   }
