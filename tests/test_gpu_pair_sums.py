@@ -1,24 +1,71 @@
 """The pair sums (pair_region) and the corner peak's group sums (group_sums)
 against the oracle at the kernel's own points, where they can go wrong: widths
-in and out of the width tables (powers of two from 1 down past the last
-table entry, and widths that are no power of two), the Gaussian's cosh table
-at its ends and past it, lists that end inside a tile and a workgroup, and
-regions out of the sums' range among regions within it.
+from 1 down past 2^-13 and widths that are no power of two, the Gaussian's cosh
+table at its ends and past it, lists that end inside a tile, and regions out of
+the sums' range among regions within it.
+
+Each flat list runs through eval_genz and as a loop's launch does
+(pagani_genz_eval_launch, _launch below), which takes the pair sums without
+tables. The level-form lists run the kernel with the
+tables: past their last level, past the cosh rows in LDS, and with an end
+inside a tile and a workgroup, bit for bit with the launches without tables.
 
 Tolerances are test_gpu_eval's: 1e-13 of each region's scale plus the FP64
 floor of f at those points, and the error and split-axis rules given there.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
 import oracle_api as O
-from test_gpu_eval import check_region_parity, genz_params, gpu_eval
+from test_gpu_eval import check_region_parity, genz_params, gpu_eval, to_dev
 
 pytestmark = pytest.mark.gpu
+
+pg = pytest.importorskip("gpuintegration_amd")
+
+
+class _Args(ctypes.Structure):  # pagani_eval_args
+    _fields_ = ([("n", ctypes.c_size_t)]
+                + [(k, ctypes.c_void_p) for k in ("L", "H", "est", "err", "dim", "stream")]
+                + [("consts", pg.EvalConsts)]
+                + [(k, ctypes.c_void_p) for k in ("dev", "L2", "H2", "pdim", "pdim2", "fevals")])
+
+
+def _launch(gpu, family, a, u, L, H, h0=None):
+    """(est, err, dim) of one launch, one wave per batch: H holds widths, or with h0 the levels of widths
+    h0 2^-level."""
+    import torch
+    d, n = L.shape
+    Ld = to_dev(np.ascontiguousarray(L.ravel()), gpu)
+    Hd = torch.from_numpy(np.ascontiguousarray(H.ravel())).to(gpu)
+    est = torch.empty(n, dtype=torch.float64, device=gpu)
+    err, dim = torch.empty_like(est), torch.empty(n, dtype=torch.uint8, device=gpu)
+    with pg.Workspace(d, 0) as ws:
+        ws.set_slices(1)
+        args = _Args(n=n, L=Ld.data_ptr(), H=Hd.data_ptr(), est=est.data_ptr(), err=err.data_ptr(),
+                     dim=dim.data_ptr())
+        rc = ws.lib.pagani_ws_eval_consts(ws._ws, None, None, n, ctypes.byref(args.consts))
+        assert (rc, args.consts.ndim, args.consts.slices) == (0, d, 1)
+        if h0 is not None:
+            assert Hd.dtype == torch.int16
+            args.consts.levels = 1
+            args.consts.h0[:d] = [h0] * d
+        torch.cuda.synchronize()
+        g = pg.genz(family, a, u)
+        assert ws.lib.pagani_genz_eval_launch(ctypes.byref(g), 64, ctypes.byref(args)) == 0
+        torch.cuda.synchronize()
+    return est.cpu().numpy(), err.cpu().numpy(), dim.cpu().numpy().astype(np.int32)
 
 
 def _compare(pg, gpu, family, a, u, L, H, slices=1):
     d, n = L.shape
+    if slices == 1 and family != "corner_peak":
+        got = _launch(gpu, family, a, u, L, H)
+        Lr, Hr = np.ascontiguousarray(L.ravel()), np.ascontiguousarray(H.ravel())
+        want = O.eval_regions_kform(d, family, O.params(a, u), Lr, Hr, n)
+        check_region_parity(d, family, *got, *want, floor=True)
     L, H = np.ascontiguousarray(L.ravel()), np.ascontiguousarray(H.ravel())
     with pg.Workspace(d, 0) as ws:
         ws.set_slices(slices)
@@ -137,3 +184,37 @@ def test_rounding_is_that_of_single_points(pg, gpu, family, d):
             est = gpu_eval(ws, gpu, family, a, u, np.ascontiguousarray(L.ravel()),
                            np.ascontiguousarray(H.ravel()), n)[0]
             assert rms(est / vol) <= 1.25 * rms(plain)
+
+
+# n = 262144 regions is the first list the kernel with tables takes; eight waves a workgroup, four with a mask
+@pytest.mark.parametrize("family", ["gaussian", "c0", "discontinuous"])
+@pytest.mark.parametrize("d,n", [(2, 262144), (2, 262144 + 64 * 5 + 1), (3, 262144 + 64 * 9 + 33),
+                                 (8, 262144 + 64 * 3 + 63)])
+@pytest.mark.parametrize("h0", [1.0, 1.0 / 3.0])
+def test_tables(pg, gpu, family, d, n, h0):
+    """A long level-form list, as doubles and in short lists the same bits; and the oracle's on a sample."""
+    rng = np.random.default_rng(7 * d + n)
+    a, u = genz_params(family, d, seed=23 + d)
+    if family == "gaussian":  # rows past the LDS part of the cosh table, and past the table
+        a[0] = 40.0
+    last = max(96 // d, 12)  # levels with a table entry: 0 .. last - 1
+    lev = rng.integers(0, last + 3, size=(d, n)).astype(np.int16)
+    lev[:, ::2] = rng.integers(0, 5, size=(d, (n + 1) // 2))
+    H = np.ldexp(h0, -lev.astype(np.int32))
+    L = np.floor(rng.random((d, n)) * (1.0 - H) / H) * H
+    assert (lev == 0).any() and (lev == last - 1).any() and (lev >= last).any()
+    if family == "gaussian":
+        row = 2 * np.abs(2 * a[0] ** 2 * (L[0] + H[0] / 2 - u[0]) * H[0])
+        assert (row < 51).any() and ((row > 51) & (row < 200)).any() and (row > 201).any()
+    long = _launch(gpu, family, a, u, L, lev, h0)
+    for part in (slice(0, 200001), slice(200001, n)):
+        for got in (_launch(gpu, family, a, u, L[:, part], lev[:, part], h0),
+                    _launch(gpu, family, a, u, L[:, part], H[:, part])):
+            for x, y in zip(long, got):
+                assert np.array_equal(x[part], y)
+    pick = np.concatenate([np.arange(300), n - 1 - np.arange(300)])
+    pick = pick[(lev[:, pick] < 12).all(0)]
+    assert pick.size > 100
+    Lp, Hp = (np.ascontiguousarray(x[:, pick].ravel()) for x in (L, H))
+    want = O.eval_regions_kform(d, family, O.params(a, u), Lp, Hp, pick.size)
+    check_region_parity(d, family, *(x[pick] for x in long), *want, floor=True)
