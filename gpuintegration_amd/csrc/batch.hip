@@ -267,11 +267,12 @@ int run_segments(pagani_batch* b, const pagani_batch_item* items, std::size_t co
         const pagani_batch_item& it = items[i];
         if (it.f.ndim != d || it.f.family != fam || it.precision != PAGANI_FP64) continue;
         if (!(it.epsrel >= 0.0) || !(it.epsabs >= 0.0)) continue;
-        // the corner peak is evaluated point by point (1105 points per 8D
-        // region, against per-axis factors for the other families): from 8D
-        // one compute unit per integral takes longer than the regular loop
-        // on the whole device (measured: 165 ms for the 8D items of the
-        // 512-integral batch, 4 ms each on the regular loop)
+        // the corner peak is evaluated at every point (1105 per 8D region,
+        // against per-axis sums for the other families): from 8D one compute
+        // unit per integral takes longer than the regular loop on the whole
+        // device (measured before the points were summed in groups, which
+        // halves both: 165 ms for the 8D items of the 512-integral batch,
+        // 4 ms each on the regular loop)
         if (fam == PAGANI_GENZ_CORNER_PEAK && d >= 8) continue;
         const std::size_t k = it.init_k ? it.init_k : I::default_split(d);
         std::size_t n = 1;

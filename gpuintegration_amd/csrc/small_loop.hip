@@ -297,7 +297,7 @@ int launch_small_part<PAGANI_PART>(hipStream_t s, const pagani_genz& g, DevLoop*
 // One compute unit issues about one wave instruction per cycle, and at two
 // waves per SIMD some 60 % of that: 40 000 instructions are 30 us, what an
 // iteration's launches cost.  Instructions per tile of 64 regions: pair sums
-// and cosine sums by axis, the corner peak by point.
+// and cosine sums by axis, the corner peak in groups of points.
 std::size_t small_cap(int family, int d)
 {
   if (d < PAGANI_MIN_DIM || d > PAGANI_GENZ_MAX_DIM) return 0;

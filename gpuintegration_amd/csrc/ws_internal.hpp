@@ -41,10 +41,6 @@ struct TraceRec {
   double estimate, errorest;
 };
 
-// State of the device-resident loop (device memory, mirrored in pinned host
-// memory between rounds).  decide_step (devloop_decide.hpp, run by the last
-// workgroup of k_step_dev) makes the host loop's per-iteration decisions on
-// it; see integrate_impl for when the loop runs on the device.
 // Iterations queued per round at most: a round that stops early leaves the
 // rest as no-op launches, so the length trades round trips for those.
 constexpr int kDevQueueMax = 16;
@@ -57,6 +53,11 @@ enum : std::int32_t {
   kDevLimit = 4,      // the iteration cap was reached after a split
 };
 
+// State of the device-resident loop (device memory, mirrored in pinned host
+// memory between rounds; the short-list loop works on the pinned copy).
+// decide_step (devloop_decide.hpp, run by the last workgroup of k_step_dev or
+// by k_small_loop) makes the host loop's per-iteration decisions on it; see
+// integrate_impl for when the loop runs on the device.
 struct DevLoop {
   pagani_dev_iter it;          // the next iteration
   pagani::phases::DevCompact cp;  // this iteration's filter + split

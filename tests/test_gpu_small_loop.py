@@ -68,7 +68,9 @@ def test_the_host_finishes_an_iteration(pg, gpu, mem):
 
 
 def test_longer_than_a_launch(pg, gpu):
-    """More iterations than the first launch takes, replayed and launched."""
+    """More iterations than the first launch (24) and the first of the later
+    ones (8) take, the others replayed and launched; every list within the
+    workgroup's (70 tiles of a 2D discontinuous integrand)."""
     for graphs in (True, False):
         a, u = [5.0, 6.0], [0.4, 0.6]
         got = []
@@ -80,4 +82,8 @@ def test_longer_than_a_launch(pg, gpu):
                     r = ws.integrate_genz("discontinuous", a, u, epsrel=1e-14, epsabs=1e-300)
                 got.append((r.estimate, r.errorest, r.nregions, r.iters, r.status,
                             list(ws.trace()["estimate"])))
+                st, sizes = ws.stats(), ws.trace()["n"]
         assert got[0] == got[1]
+        assert max(sizes) <= 70 * 64 and len(sizes) > 24 + 8
+        assert st["device_iterations"] == 2 * len(sizes)
+        assert st["graph_launches"] == (2 * (-(-(len(sizes) - 24) // 8) - 1) if graphs else 0)
