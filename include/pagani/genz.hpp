@@ -308,8 +308,8 @@ struct ProductPeak {
   // quotient by its remainder (not of lambda4's, which weighs in a null rule
   // only): the sum rounds as two factors one by one do.  Without it a region's
   // error is 1.1 to 1.2 times theirs, 2D to 5D; 8D, 10^6 regions: 54 -> 56 us,
-  // one by one 110.  |v|, |h| <= 1e7 keeps that product, and the centre's prod_j A,
-  // below 1e150.
+  // one by one 110.  |v|, |h| <= 1e13 keeps that product (of twenty numbers
+  // up to 1.5e13), and the centre's prod_j A (ten of 1e26), below 1e265.
   struct Centre {
     double den = 1.0, big = 0.0;
     __device__ void add(const ProductPeak&, int, double c, double h)
@@ -317,7 +317,7 @@ struct ProductPeak {
       den *= __builtin_fma(c, c, 1.0);
       big = __builtin_fmax(big, __builtin_fmax(__builtin_fabs(c), __builtin_fabs(h)));
     }
-    __device__ bool safe(const ProductPeak&) const { return big <= 1e7; }
+    __device__ bool safe(const ProductPeak&) const { return big <= 1e13; }
     __device__ double value(const ProductPeak& f) const { return f.k2 / den; }
   };
   static constexpr int kWidthValues = 0, kTableSize = 0;

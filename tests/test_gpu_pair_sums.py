@@ -106,6 +106,17 @@ def test_gaussian_at_the_ends_of_its_table(pg, gpu, d):
     _compare(pg, gpu, "gaussian", a, u, L, H)
 
 
+@pytest.mark.parametrize("d", [2, 3, 10])
+@pytest.mark.parametrize("first", [1e8, 4e13, 1e16])
+def test_product_peak_at_the_end_of_its_range(pg, gpu, d, first):
+    # v = a (x - u) up to 1e13 is within the pair sums' range; 4e13 has regions on both sides
+    n = 64 * 5 + 3
+    rng = np.random.default_rng(d)
+    a, u = [first] + [9.0] * (d - 1), [0.4] * d
+    H = 0.5 ** rng.integers(1, 9, size=(d, n))
+    _compare(pg, gpu, "product_peak", a, u, _boxes(rng, H), H)
+
+
 @pytest.mark.parametrize("d", [2, 3, 5, 8])
 @pytest.mark.parametrize("slices", [1, 2, 4, 8])
 @pytest.mark.parametrize("first", [9.0, 1e31])
