@@ -1535,9 +1535,9 @@ constexpr std::size_t kPairLong = 4096;
 
 // Kernel: the evaluation of a has_pair_sums integrand on a level-form list at
 // one wave per tile of 64 regions (slices == 1), with its tables.  Bound by
-// vector issue (8D Gaussian, 31.5 M regions: 1 592 instructions a region, 88 %
-// of the issue rate; 1.45 ms a launch against 2.15-2.22 for the factored sums
-// with two factors per axis and magnitude).
+// vector issue (8D Gaussian, 31.5 M regions: 1 592 instructions a region, 86 to
+// 88 % of the issue rate; 1.45-1.49 ms a launch against 2.15-2.22 for the
+// factored sums with two factors per axis and magnitude).
 template <int D, class F>
 __global__ void __launch_bounds__(64 * kPairWaves<F>, kPairPerSimd<F>)
     pair_kernel(F f, const pagani_dev_iter* __restrict__ it, std::size_t n_arg,
