@@ -7,9 +7,9 @@
 // each), the ticket of k_step_dev with its device-wide fences (17-45 us),
 // queued launches after the loop had stopped, and a round trip per round.
 // Measured per integral, as those launches -> here: 5D oscillatory at 1e-3
-// (one iteration of 32 regions, eight waves on their one tile) 65 -> 48 us; 3D Gaussian at 1e-4 443 -> 267 us, 5D discontinuous at
-// 1e-4 2.07 -> 1.36 ms (228 us and 1.18 ms with the shorter k_step_dev on the
-// lists past small_cap).
+// (one iteration of 32 regions, eight waves on their one tile) 65 -> 48 us; 3D
+// Gaussian at 1e-4 443 -> 267 us, 5D discontinuous at 1e-4 2.07 -> 1.36 ms (228
+// us and 1.18 ms with the shorter k_step_dev on the lists past small_cap).
 // Here one workgroup of 512 threads runs the whole loop: uniform barriers in
 // place of launches, the loop's state and the sums in LDS, the lists in the
 // workspace's own buffers (so the loop can stop at any iteration and the
