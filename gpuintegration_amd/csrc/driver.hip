@@ -1455,7 +1455,7 @@ int pagani_eval_genz_dev(pagani_ws* ws, const pagani_genz* f, int precision, siz
   ws->tune_precision = precision;
   make_consts(ws, lows, highs, n, args.consts);
   record(ws, EV_EVAL0);
-  rc = genz_eval(f, precision, &args, true);
+  rc = pagani_genz_eval_launch(f, precision, &args);
   if (rc) return fail(ws, rc, "evaluation launch failed");
   record(ws, EV_EVAL1);
   HIP_TRY(ws, hipStreamSynchronize(ws->stream));

@@ -16,15 +16,15 @@ namespace pagani {
 namespace internal {
 
 template <class Real, int D>
-int genz_launch(const pagani_genz* g, const pagani_eval_args* a, bool own_list)
+int genz_launch(const pagani_genz* g, const pagani_eval_args* a)
 {
   return visit_genz<Real, D>(g, [&](const auto& f) {
-    return pagani::eval_regions<D, std::decay_t<decltype(f)>, Real>(f, a, own_list);
+    return pagani::eval_regions<D, std::decay_t<decltype(f)>, Real>(f, a);
   });
 }
 
 #define PAGANI_GENZ(Real, D) \
-  template int genz_launch<Real, D>(const pagani_genz*, const pagani_eval_args*, bool);
+  template int genz_launch<Real, D>(const pagani_genz*, const pagani_eval_args*);
 #if PAGANI_PART == 0
 PAGANI_GENZ(double, 2)
 PAGANI_GENZ(double, 3)
@@ -53,7 +53,7 @@ PAGANI_GENZ(float, 9)
 
 #if PAGANI_PART == 0
 #define PAGANI_GENZ_ELSEWHERE(Real, D) \
-  extern template int genz_launch<Real, D>(const pagani_genz*, const pagani_eval_args*, bool);
+  extern template int genz_launch<Real, D>(const pagani_genz*, const pagani_eval_args*);
 PAGANI_GENZ_ELSEWHERE(double, 6)
 PAGANI_GENZ_ELSEWHERE(double, 7)
 PAGANI_GENZ_ELSEWHERE(double, 8)
@@ -70,28 +70,20 @@ PAGANI_GENZ_ELSEWHERE(float, 9)
 PAGANI_GENZ_ELSEWHERE(float, 10)
 
 template <class Real>
-int launch_dim(const pagani_genz* g, const pagani_eval_args* a, bool own_list)
+int launch_dim(const pagani_genz* g, const pagani_eval_args* a)
 {
   switch (g->ndim) {
-  case 2: return genz_launch<Real, 2>(g, a, own_list);
-  case 3: return genz_launch<Real, 3>(g, a, own_list);
-  case 4: return genz_launch<Real, 4>(g, a, own_list);
-  case 5: return genz_launch<Real, 5>(g, a, own_list);
-  case 6: return genz_launch<Real, 6>(g, a, own_list);
-  case 7: return genz_launch<Real, 7>(g, a, own_list);
-  case 8: return genz_launch<Real, 8>(g, a, own_list);
-  case 9: return genz_launch<Real, 9>(g, a, own_list);
-  case 10: return genz_launch<Real, 10>(g, a, own_list);
+  case 2: return genz_launch<Real, 2>(g, a);
+  case 3: return genz_launch<Real, 3>(g, a);
+  case 4: return genz_launch<Real, 4>(g, a);
+  case 5: return genz_launch<Real, 5>(g, a);
+  case 6: return genz_launch<Real, 6>(g, a);
+  case 7: return genz_launch<Real, 7>(g, a);
+  case 8: return genz_launch<Real, 8>(g, a);
+  case 9: return genz_launch<Real, 9>(g, a);
+  case 10: return genz_launch<Real, 10>(g, a);
   default: return PAGANI_EUNSUPPORTED;
   }
-}
-
-int genz_eval(const pagani_genz* g, int precision, const pagani_eval_args* a, bool own_list)
-{
-  if (!g || !a) return PAGANI_EBADARG;
-  if (precision == PAGANI_FP64) return launch_dim<double>(g, a, own_list);
-  if (precision == PAGANI_FP32) return launch_dim<float>(g, a, own_list);
-  return PAGANI_EBADARG;
 }
 #endif
 
@@ -102,6 +94,9 @@ int genz_eval(const pagani_genz* g, int precision, const pagani_eval_args* a, bo
 extern "C" int pagani_genz_eval_launch(const pagani_genz* g, int precision,
                                        const pagani_eval_args* a)
 {
-  return pagani::internal::genz_eval(g, precision, a, false);
+  if (!g || !a) return PAGANI_EBADARG;
+  if (precision == PAGANI_FP64) return pagani::internal::launch_dim<double>(g, a);
+  if (precision == PAGANI_FP32) return pagani::internal::launch_dim<float>(g, a);
+  return PAGANI_EBADARG;
 }
 #endif

@@ -13,12 +13,4 @@ int pagani_genz_eval_launch(const pagani_genz* f, int precision, const pagani_ev
 
 #ifdef __cplusplus
 }
-
-namespace pagani {
-namespace internal {
-// The same; own_list: a caller's flat list, which no loop's launches go on from.
-int genz_eval(const pagani_genz* g, int precision, const pagani_eval_args* a, bool own_list);
-}  // namespace internal
-}  // namespace pagani
-
 #endif

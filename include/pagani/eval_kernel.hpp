@@ -1250,7 +1250,7 @@ __device__ __forceinline__ double point_generator(const pagani_eval_consts& C, i
 // == 1); with more than one, every wave of the workgroup passes one barrier,
 // and only wave 0 returns true (holding the results).  `lows`, `range`,
 // `jac` describe the integration box.
-template <int D, class F, class Real, bool Pairs, bool FusedAngle, bool Factors>
+template <int D, class F, class Real, bool Pairs, bool FusedAngle>
 __device__ __forceinline__ bool eval_region_values(
     F& f, const double* __restrict__ L, const double* __restrict__ H,
     const std::uint8_t* __restrict__ pdim, std::size_t n, std::size_t t,
@@ -1275,7 +1275,7 @@ __device__ __forceinline__ bool eval_region_values(
   }
   if constexpr (has_group_sums<F>::value) {
     done = group_sums<D, F>(f, cR, hR, C, slices, wave, rs, bisect);
-  } else if constexpr (has_pair_sums<F>::value && !Factors) {
+  } else if constexpr (has_pair_sums<F>::value) {
     // a region out of the pair sums' range, and several waves: the generic loop
   } else if constexpr (is_cosine<F>::value && has_origin<F>::value && has_axis_scale<F>::value) {
     if (slices == 1) done = cosine_sums<D, F, Real>(f, angle, hR, jac, C, rs, bisect);
@@ -1394,7 +1394,7 @@ __device__ __forceinline__ bool eval_region_values(
 }
 
 // eval_region_values, stored: region t's estimate, error and split axis.
-template <int D, class F, class Real, bool Pairs, bool FusedAngle = false, bool Factors = false>
+template <int D, class F, class Real, bool Pairs, bool FusedAngle = false>
 __device__ __forceinline__ void eval_regions_wave(
     F& f, const double* __restrict__ L, const double* __restrict__ H,
     const std::uint8_t* __restrict__ pdim, std::size_t n, std::size_t t, bool live,
@@ -1404,9 +1404,9 @@ __device__ __forceinline__ void eval_regions_wave(
 {
   double avg, er;
   int axis;
-  if (!eval_region_values<D, F, Real, Pairs, FusedAngle, Factors>(
-          f, L, H, pdim, n, t, lows, range, jac, C, slices, wave, lane, part, row, tab, avg, er,
-          axis))
+  if (!eval_region_values<D, F, Real, Pairs, FusedAngle>(f, L, H, pdim, n, t, lows, range, jac, C,
+                                                         slices, wave, lane, part, row, tab, avg,
+                                                         er, axis))
     return;
   if (live) {
     est[t] = avg;
@@ -1477,9 +1477,8 @@ struct LaunchList {
 // iteration's slice count only keep the barrier company.  Host-driven and
 // device-loop launches run this one kernel, so a given n and slice count
 // give the same bits either way.  Dynamic LDS: (waves per workgroup -
-// 1)*5*64 doubles.  Pairs: the pair sums without tables (slices == 1);
-// Factors: a pair-sum integrand by its factors one by one (slices == 1).
-template <int D, class F, class Real, bool Pairs, bool Factors = false>
+// 1)*5*64 doubles.  Pairs: the pair sums without tables (slices == 1).
+template <int D, class F, class Real, bool Pairs>
 __global__ void __launch_bounds__(64 * PAGANI_MAX_SLICES)
     eval_kernel(F f, const pagani_dev_iter* __restrict__ it, std::size_t n_arg,
                 const double* __restrict__ L0, const double* __restrict__ H0,
@@ -1512,9 +1511,9 @@ __global__ void __launch_bounds__(64 * PAGANI_MAX_SLICES)
                                                 C.range, C.jac, C, 1, 0, lane, nullptr, &row,
                                                 nullptr, est, err, dim);
   } else {
-    detail::eval_regions_wave<D, F, Real, false, false, Factors>(
-        f, list.L, list.H, list.P, list.n, t, live, C.lows, C.range, C.jac, C, list.slices, wave,
-        lane, part, nullptr, nullptr, est, err, dim);
+    detail::eval_regions_wave<D, F, Real, false>(f, list.L, list.H, list.P, list.n, t, live,
+                                                 C.lows, C.range, C.jac, C, list.slices, wave,
+                                                 lane, part, nullptr, nullptr, est, err, dim);
   }
 }
 
@@ -1600,10 +1599,8 @@ __global__ void __launch_bounds__(256)
 
 // Launch the evaluation of args->n regions for integrand f.  Returns 0 or
 // PAGANI_EHIP.  Real is the integrand's arithmetic type (double or float).
-// own_list: a caller's flat list, no list of a loop whose other launches have
-// to form the same bits.
 template <int D, class F, class Real = double>
-int eval_regions(const F& f, const pagani_eval_args* args, bool own_list = false)
+int eval_regions(const F& f, const pagani_eval_args* args)
 {
   static_assert(D >= PAGANI_MIN_DIM && D <= PAGANI_MAX_DIM, "unsupported ndim");
   // a library built from other headers lays its lists out differently
@@ -1635,19 +1632,7 @@ int eval_regions(const F& f, const pagani_eval_args* args, bool own_list = false
       const int pw = kPairWaves<F>;
       if (tables) launch(pair_kernel<D, F>, (tiles + pw - 1) / pw, 64 * pw, 0);
     }
-    // A caller's flat list has widths of its own, so a region's width values
-    // are formed for it alone and the pair sums spare nothing on a short list:
-    // 3 000 regions at 8D, Gaussian 24.2 us a call with them, 22.4 by factors,
-    // C0 23.3 and 22.1. On long ones they do without a mask (C0, 10^6 regions:
-    // 8D 79 against 82 us, 5D 59 against 61) and, for the Gaussian, whose rows
-    // come from memory, up to 5D (5D 62 against 63.5 us, 8D 89 against 86).
-    bool factors = false;
-    if constexpr (detail::pair_table_size<D, F>() > 0) {
-      constexpr bool kLongPairs = !detail::is_masked<F>::value && (F::kTableSize == 0 || D <= 5);
-      factors = pairs && own_list && !(kLongPairs && tiles >= kPairLong);
-      if (factors) launch(eval_kernel<D, F, Real, false, true>, tiles, 64, 0);
-    }
-    if (pairs && !tables && !factors) launch(eval_kernel<D, F, Real, true>, tiles, 64, 0);
+    if (pairs && !tables) launch(eval_kernel<D, F, Real, true>, tiles, 64, 0);
   }
   if (!pairs)
     launch(eval_kernel<D, F, Real, false>, tiles, 64 * waves,

@@ -644,35 +644,6 @@ struct C0 {
       }
     }
   }
-  // The points v -+ delta of one axis change |v| by -+delta when they stay
-  // on v's side of the kink: factors e^delta (toward 0) and e^-delta (away),
-  // one exponential and its reciprocal.  A point across the kink (delta >
-  // |v|) has e^(2|v| - delta) = (e^-delta e^|v|) e^|v|, with aux = e^|v|
-  // (|v| <= 650 where the factored form is taken, so aux stays finite and
-  // the first product is at most 1).
-  // (FP64 integrands only: for an FP32 one the extra registers cost more
-  // than the exponentials they save)
-  template <class R = Real, if_double<R> = 0>
-  __device__ double axis_aux(int, double v) const
-  {
-    return math::exp_factor(__builtin_fabs(v), Real());
-  }
-  template <class R = Real, if_double<R> = 0>
-  __device__ void factor_pair(int, double v, double delta, double aux, double& fm,
-                              double& fp) const
-  {
-    const double e = math::exp_factor(-delta, Real());
-    const double r = math::recip(e);
-    const double across = (e * aux) * aux;
-    const bool cross = delta > __builtin_fabs(v);
-    if (v >= 0.0) {
-      fm = cross ? across : r;
-      fp = e;
-    } else {
-      fm = e;
-      fp = cross ? across : r;
-    }
-  }
   // outer(s + d) = outer(s) e^-d, non-negative terms (see Gaussian)
   static constexpr bool exponential = true;
   __device__ double factor(double d) const { return math::exp_factor(-d, Real()); }

@@ -4,10 +4,9 @@ from 1 down past 2^-13 and widths that are no power of two, the Gaussian's cosh
 table at its ends and past it, lists that end inside a tile, and regions out of
 the sums' range among regions within it.
 
-A caller's short list of the families with width values takes their factors one
-by one instead, so each flat list here runs both ways: through eval_genz and
-as a loop's launch does (pagani_genz_eval_launch, _launch below), which takes
-the pair sums without tables. The level-form lists run the kernel with the
+Each flat list runs through eval_genz and as a loop's launch does
+(pagani_genz_eval_launch, _launch below), which takes the pair sums without
+tables. The level-form lists run the kernel with the
 tables: past their last level, past the cosh rows in LDS, and with an end
 inside a tile and a workgroup, bit for bit with the launches without tables.
 
@@ -230,26 +229,3 @@ def test_tables(pg, gpu, family, d, n, h0):
     Lp, Hp = (np.ascontiguousarray(x[:, pick].ravel()) for x in (L, H))
     want = O.eval_regions_kform(d, family, O.params(a, u), Lp, Hp, pick.size)
     check_region_parity(d, family, *(x[pick] for x in long), *want, floor=True)
-
-
-@pytest.mark.parametrize("family", ["gaussian", "c0", "discontinuous"])
-@pytest.mark.parametrize("d", [2, 5, 8])
-def test_long_lists_of_a_caller(pg, gpu, family, d):
-    """262144 regions of a caller's, where the rule between pair sums and factors turns, against the halves."""
-    n = 262144 + 65
-    rng = np.random.default_rng(d)
-    a, u = genz_params(family, d, seed=5 + d)
-    H = 0.5 ** rng.integers(1, 8, size=(d, n))
-    L = _boxes(rng, H)
-    with pg.Workspace(d, 0) as ws:
-        ws.set_slices(1)
-        ev = lambda s: gpu_eval(ws, gpu, family, a, u, np.ascontiguousarray(L[:, s].ravel()),  # noqa: E731
-                                np.ascontiguousarray(H[:, s].ravel()), L[:, s].shape[1])
-        whole, parts = ev(slice(0, n)), [ev(slice(0, n // 2)), ev(slice(n // 2, n))]
-    est = np.concatenate([p[0] for p in parts])
-    # each is within 1e-13 of the sum of its terms' magnitudes
-    w, _, _, _, sb, _ = pg.rule_tables(d)
-    terms = sum(abs(w[k][0]) * (sb[k + 1] - sb[k]) for k in range(9))
-    top = np.exp((np.array(a)[:, None] * np.minimum(L + H, np.array(u)[:, None])).sum(0)) \
-        if family == "discontinuous" else 1.0
-    assert (np.abs(whole[0] - est) <= 2e-13 * terms * top * H.prod(0)).all()
