@@ -6,8 +6,8 @@ the sums' range among regions within it.
 
 Each flat list runs through eval_genz and as a loop's launch does
 (pagani_genz_eval_launch, _launch below), which takes the pair sums without
-tables. The level-form lists run the kernel with the
-tables: past their last level, past the cosh rows in LDS, and with an end
+tables. The level-form lists run the kernel with the tables: past their last
+level, past the cosh rows in LDS, and with an end
 inside a tile and a workgroup, bit for bit with the launches without tables.
 
 Tolerances are test_gpu_eval's: 1e-13 of each region's scale plus the FP64
