@@ -205,8 +205,8 @@ __device__ bool refine_axis(const double* __restrict__ hist, const double* xi, d
 }
 
 __global__ void __launch_bounds__(kStepThreads)
-    k_mc_step(int d, int hist_dims, int it, int slot, int joins, double dv2g, double epsrel, double epsabs,
-              const double* __restrict__ out, double* xi, double* state)
+    k_mc_step(int d, int hist_dims, int it, int slot, int joins, double dv2g, double epsrel,
+              double epsabs, const double* __restrict__ out, double* xi, double* state)
 {
   if (state[kLive] == 0.0) return;
   if (blockIdx.x == 0 && threadIdx.x == blockDim.x - 1) {  // a thread without a bin
@@ -392,15 +392,17 @@ int run(pagani_mc* mc, pagani_mc_sample_fn sample, void* ctx, int queue, double 
       const bool adjusts = it <= p.adjust_iters;
       a.hist_dims = adjusts ? static_cast<std::uint32_t>(hd) : 0;
       a.key = pagani::mc::iter_key(p.seed, it);
-      if ((rc = queue_pass(mc, sample, ctx, a))) {
+      if (!(rc = queue_pass(mc, sample, ctx, a))) {
+        hipLaunchKernelGGL(k_mc_step, dim3(adjusts ? hd : 1), dim3(adjusts ? kStepThreads : 64), 0,
+                           mc->stream, d, static_cast<int>(a.hist_dims), it, it - first,
+                           !adjusts || it > p.skip_iters ? 1 : 0, s.dv2g, epsrel, epsabs,
+                           mc->d_out, mc->d_xi, state);
+        if (hipGetLastError() != hipSuccess) rc = fail(mc, PAGANI_EHIP, "k_mc_step launch failed");
+      }
+      if (rc) {
         (void)hipStreamSynchronize(mc->stream);  // h_xi is the next run's
         return rc;
       }
-      hipLaunchKernelGGL(k_mc_step, dim3(adjusts ? hd : 1), dim3(adjusts ? kStepThreads : 64), 0,
-                         mc->stream, d, static_cast<int>(a.hist_dims), it, it - first,
-                         !adjusts || it > p.skip_iters ? 1 : 0, s.dv2g, epsrel, epsabs, mc->d_out,
-                         mc->d_xi, state);
-      MC_TRY(mc, hipGetLastError());
     }
     // the state, and with it the grid
     MC_TRY(mc, hipMemcpyAsync(mc->h_xi, mc->d_xi, (xi.size() + kStateDoubles) * sizeof(double),

@@ -1058,12 +1058,14 @@ int mc_dispatch(const char* name, int mode, double epsrel, double ncall, int tit
 
 // A run whose callback counts its calls and passes on its own arguments, as a
 // program with a sampler of its own may: *calls and *out.
+// fails > 0: a first run's callback fails at that call, its code in *first;
+// then the run is made on the same handle.
 extern "C" int reftest_mc_calls(double epsrel, double ncall, int titer, int itmax, int skip,
-                                int* calls, pagani_mc_result* out)
+                                int fails, int* first, int* calls, pagani_mc_result* out)
 {
   struct Ctx {
     Gauss1D f;
-    int calls;
+    int calls, fails;
   } ctx{};
   pagani_mc* mc = pagani_mc_create(1, -1);
   if (!mc) return -1;
@@ -1073,14 +1075,21 @@ extern "C" int reftest_mc_calls(double epsrel, double ncall, int titer, int itma
   p.adjust_iters = itmax;
   p.skip_iters = skip;
   p.generator = PAGANI_MC_RNG_DEFAULT;
-  const int rc = pagani_mc_integrate_cb(
-      mc,
-      [](void* c, const pagani_mc_args* a) {
-        Ctx* x = static_cast<Ctx*>(c);
-        x->calls++;
-        return pagani::mc::launch<1, Gauss1D, pagani::mc::XoroStream>(x->f, a);
-      },
-      &ctx, epsrel, 1e-30, nullptr, nullptr, &p, out);
+  auto sample = [](void* c, const pagani_mc_args* a) -> int {
+    Ctx* x = static_cast<Ctx*>(c);
+    if (++x->calls == x->fails) return PAGANI_EUNSUPPORTED;
+    return pagani::mc::launch<1, Gauss1D, pagani::mc::XoroStream>(x->f, a);
+  };
+  auto run = [&] {
+    return pagani_mc_integrate_cb(mc, sample, &ctx, epsrel, 1e-30, nullptr, nullptr, &p, out);
+  };
+  *first = 0;
+  if (fails > 0) {
+    ctx.fails = fails;
+    *first = run();
+    ctx = Ctx{};
+  }
+  const int rc = run();
   *calls = ctx.calls;
   pagani_mc_destroy(mc);
   return rc;

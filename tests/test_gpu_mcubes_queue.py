@@ -73,13 +73,28 @@ def _reftests():
     return ctypes.CDLL(os.path.join(os.path.dirname(os.path.abspath(__file__)), "cxx", "libreftests.so"))
 
 
+def _callback_run(eps, total, adjust, fails=0):
+    first, calls, r = ctypes.c_int(), ctypes.c_int(), pg.McResult()
+    rc = _reftests().reftest_mc_calls(ctypes.c_double(eps), ctypes.c_double(2e4), total, adjust, 0, fails,
+                                      ctypes.byref(first), ctypes.byref(calls), ctypes.byref(r))
+    assert rc == 0
+    return first.value, calls.value, r
+
+
 @pytest.mark.parametrize("eps,total,adjust,iters", [(1e-12, 20, 4, 20), (0.5, 40, 3, 5), (0.5, 40, 20, 5)])
 def test_callback_is_called_once_per_iteration(gpu, eps, total, adjust, iters):
     """A callback need not know of iterations queued ahead: it sees the run's own, no more."""
-    calls, r = ctypes.c_int(), pg.McResult()
-    rc = _reftests().reftest_mc_calls(ctypes.c_double(eps), ctypes.c_double(2e4), total, adjust, 0,
-                                      ctypes.byref(calls), ctypes.byref(r))
-    assert (rc, r.iters, calls.value) == (0, iters, iters)
+    calls, r = _callback_run(eps, total, adjust)[1:]
+    assert (r.iters, calls) == (iters, iters)
+
+
+def test_a_failing_callback_leaves_the_handle_usable(gpu):
+    """The run after one whose callback failed in its third iteration is the run of a fresh handle (no
+    adjusting iterations: those repeat to the last bits only, their histograms being LDS additions)."""
+    first, calls, r = _callback_run(1e-12, 8, 0, fails=3)
+    fresh = _callback_run(1e-12, 8, 0)[2]
+    assert first == pg.EUNSUPPORTED and calls == 8
+    assert (r.estimate, r.errorest, r.iters, r.status) == (fresh.estimate, fresh.errorest, 8, 1)
 
 
 def test_own_grid_ends_with_its_last_edge(gpu):
